@@ -210,16 +210,12 @@ extern "C" int lag_hip_sync(void) {
 }
 
 // The grouped expert GEMMs of a batch: dot8 (k_dot8.hip) or the f16 MFMA
-// (k_mfma.hip), bit-identical; auto takes the MFMA when the groups average at
-// least 6.5 tokens (SW_MF_MIN_AVG2 / 2).  Measured on the C2 layer (dot8 against MFMA
-// per step): B=160 1,009 against 1,055 us, B=176 1,088 against 1,065, B=192 1,167 against
-// 1,072, B=256 1,476 against 1,105.
+// (k_mfma.hip), bit-identical; auto takes the MFMA where it wins (sw_mf_wins, sw_hip.h).
 static int g_grouped_kernel = 0;        // 0 auto, 1 dot8, 2 MFMA
-#define SW_MF_MIN_AVG2 13
 static bool use_mfma(int T, int E, int D, int I) {
     if (g_grouped_kernel == 1 || D % 128 || I % 128) return false;      // whole chunks of 4 input groups
     if (g_grouped_kernel == 2) return true;
-    return 2 * (int64_t)T >= SW_MF_MIN_AVG2 * (int64_t)(T < E ? T : E);
+    return sw_mf_wins(T, T < E ? T : E);
 }
 extern "C" int lag_hip_set_grouped_kernel(int mode) {
     if (mode < 0 || mode > 2) return -1;
@@ -263,9 +259,10 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
     if (!g_ok || fault_injected()) return -1;
     if (D <= 0 || I <= 0 || G <= 0 || S <= 0) return -1;
     const int T = S * K;
-    // the MFMA kernels for prefill-sized groups: tiles of up to 64 tokens, listed here
+    // the MFMA kernels for prefill-sized groups: tiles of up to tt tokens, listed here
+    const int tt = sw_mf_cols(T, G);
     int ntile = 0;
-    for (int i = 0; i < G; i++) ntile += (gcnt[i] + SW_MF_TT - 1) / SW_MF_TT;
+    for (int i = 0; i < G; i++) ntile += (gcnt[i] + tt - 1) / tt;
     const bool mf = G < 1024 && T < (1 << 21) && use_mfma(T, G, D, I);
     Carve cv;
     const size_t idxn = (size_t)(3 * G + 2 * T) * 4 + (size_t)T * 4 + (mf ? (size_t)(ntile + 1) * 4 : 0);
@@ -292,7 +289,7 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
     if (mf) {
         int *it = hi + 3 * G + 3 * T, n = 0;
         for (int i = 0; i < G; i++)
-            for (int t0 = 0; t0 < gcnt[i]; t0 += sw_mf_tile(gcnt[i])) it[n++] = (t0 << 10) | i;
+            for (int t0 = 0; t0 < gcnt[i]; t0 += sw_mf_tile(gcnt[i], tt)) it[n++] = (t0 << 10) | i;
         it[n] = n;
     }
     CK(hipMemcpyAsync(A + o_x, H, xn, hipMemcpyHostToDevice, g_st), "x upload");
@@ -312,7 +309,7 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
     for (int i = 0; i < G; i++) maxcnt = gcnt[i] > maxcnt ? gcnt[i] : maxcnt;
     if (mf) {
         const int *d_items = (const int *)(d_w + T);
-        const SwGroups gt = {d_gexp, d_gbeg, d_gcnt, d_grow, nullptr, ntile, 0, d_items, d_items + ntile};
+        const SwGroups gt = {d_gexp, d_gbeg, d_gcnt, d_grow, nullptr, ntile, 0, d_items, d_items + ntile, tt};
         SwGroups gd = gt;
         gd.grow = nullptr;
         uint32_t *xd = (uint32_t *)(A + o_xd), *hd = (uint32_t *)(A + o_hd);
@@ -782,12 +779,13 @@ static int forward(const LagHipMoeDesc *d, const LagHipMoeWeights *w, const floa
               return fail_msg("down/combine launch"); }
         g_last_G_dev = 0; g_last_ng = K;
     } else if (mf) {                     // prefill: tiles of up to 64 tokens of a group on the f16 MFMA
+        const int tt = sw_mf_cols(T, T < E ? T : E);
         { PROF("bucket");
           // (the split sort's counts in the slots, which the down launch writes later)
-          if (sw_launch_bucket(g_st, f.sel, S, K, E, f.gexp, f.gbeg, f.gcnt, f.G, f.grow, f.rowof, SW_MF_TT, f.items, f.P,
+          if (sw_launch_bucket(g_st, f.sel, S, K, E, f.gexp, f.gbeg, f.gcnt, f.G, f.grow, f.rowof, tt, f.items, f.P,
                                (int *)f.slots))
               return fail_msg("bucket launch"); }
-        SwGroups g = {f.gexp, f.gbeg, f.gcnt, f.grow, f.G, sw_npass_max(T, E, SW_MF_TT), 0, f.items, f.P};
+        SwGroups g = {f.gexp, f.gbeg, f.gcnt, f.grow, f.G, sw_npass_max(T, E, tt), 0, f.items, f.P, tt};
         { PROF("mf_glu");
           if (sw_launch_mf_glu(g_st, gu, f.xd, f.xds, S, g, I, f.hd, f.hds)) return fail_msg("MFMA gate_up launch"); }
         if (sh) {

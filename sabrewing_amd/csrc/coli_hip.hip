@@ -170,8 +170,8 @@ GLay glay(const Groups &G, int T, int xrows, int nextra = 0, bool mf = false) {
     L.end = cv.off;
     return L;
 }
-// the f16 MFMA GEMMs for prefill-sized groups (16-token tiles mostly full), as
-// the lag family's automatic choice: whole chunks of 4 input groups, >= 8 rows per group
+// the f16 MFMA GEMMs from 8 rows a group on (the lag family's groups are many, and take them
+// from fewer): whole quads of 4 input groups
 bool use_mf(const Groups &G) { return G.D % 128 == 0 && G.I % 128 == 0 && G.total >= 8 * G.count; }
 size_t meta_bytes(const Groups &G, int T) { return (size_t)(3 * G.count + T) * 4 + (size_t)G.count * sizeof(SwTab); }
 // the host image of the ints and the table: gexp = 0..count-1 (the table index),
@@ -208,13 +208,13 @@ void count_group(const Groups &G) {
     g_grows += (uint64_t)G.total;
 }
 
-// the MFMA form of the group: digits of x, gate/up + GLU, down, over 64-token tiles
+// the MFMA form of the group: digits of x, gate/up + GLU, down, over tiles of tt tokens
 // (items[j] = (t0 << 10) | group, then their count) listed after gexp gbeg gcnt
-int launch_group_mf(Ctx *c, const Groups &G, char *A, const GLay &L, int ntile) {
+int launch_group_mf(Ctx *c, const Groups &G, char *A, const GLay &L, int ntile, int tt) {
     const int *d = (const int *)(A + L.ints);
     const int *items = d + 3 * G.count;
     const SwTab *tab = (const SwTab *)(A + L.tab);
-    const SwGroups gt = {d, d + G.count, d + 2 * G.count, nullptr, nullptr, ntile, 0, items, items + ntile};
+    const SwGroups gt = {d, d + G.count, d + 2 * G.count, nullptr, nullptr, ntile, 0, items, items + ntile, tt};
     const SwQ4 gu = {nullptr, nullptr, 2 * G.I, G.D, G.gs_gu, 1};
     const SwQ4 dn = {nullptr, nullptr, G.D, G.I, G.gs_d, 1};
     uint32_t *xd = (uint32_t *)(A + L.xl), *hd = (uint32_t *)(A + L.hl);
@@ -233,10 +233,11 @@ int group_sync(const Groups &G, float *y, const float *x) {
     if (!select_ctx(c)) return 0;
     const int T = G.total;
     const bool mf = use_mf(G);
+    const int tt = sw_mf_cols(T, G.count);                 // tokens per MFMA tile
     std::vector<int> items;
     if (mf) {
         for (int g = 0; g < G.count; g++)
-            for (int t0 = 0; t0 < G.cnt[g]; t0 += sw_mf_tile(G.cnt[g])) items.push_back((t0 << 10) | g);
+            for (int t0 = 0; t0 < G.cnt[g]; t0 += sw_mf_tile(G.cnt[g], tt)) items.push_back((t0 << 10) | g);
         items.push_back((int)items.size());
     }
     const int ni = (int)items.size();
@@ -265,7 +266,7 @@ int group_sync(const Groups &G, float *y, const float *x) {
             "expert group table"))
         return 0;
     if (prof) (void)hipEventRecord(c->prof[1], c->st);
-    if (mf ? !launch_group_mf(c, G, A, L, ni - 1) : !launch_group(c, G, A, L, T, T, false)) return 0;
+    if (mf ? !launch_group_mf(c, G, A, L, ni - 1, tt) : !launch_group(c, G, A, L, T, T, false)) return 0;
     if (prof) (void)hipEventRecord(c->prof[2], c->st);
     if (!ok(hipMemcpyAsync(c->hout, A + L.y, xb, hipMemcpyDeviceToHost, c->st), "expert group output download")) return 0;
     if (prof) (void)hipEventRecord(c->prof[3], c->st);

@@ -23,52 +23,46 @@
 // the slot order of mf_expand), and its A operand holds the same inputs of a
 // weight row as f16, expanded from packed dword q of the row's group.
 //
-// Block: 128 weight rows (8 tiles of 16) x a tile of up to 64 tokens (4
-// tiles of 16) of one group, 16 waves; wave w takes row tiles w&3 and (w&3)+4
-// (for gate_up the gate and the up rows of the same 16 outputs) against
-// token tile w>>2, so each lane holds 8 (row, token) sums and a wave stays
-// within 128 registers: four waves per SIMD, which hide each other's MFMA,
-// LDS and barrier waits.  The operands of 4 input groups at a time -- the
-// rows' weights expanded once for the 16 waves, the tokens' digits, the
-// scales and the token factors -- are staged in LDS in two buffers: while the
-// waves compute one chunk from LDS, the next chunk's loads are in flight in
-// registers, issued before each chunk's barrier so that the waves waiting there
-// overlap them.  Each staging wave load covers 16 rows (or tokens) with the
-// chunk's 4 groups side by side in memory: 16 cache lines a load, not 64 (the
-// staging loads' cache lines, more than the VALU, set the chunk's time).  A
-// tile's token tiles with no tokens compute nothing and have no digits staged;
-// a group's tokens are split into equal tiles of whole 16-token columns
-// (sw_mf_tile).  The inner loop reads LDS only, every wave read a contiguous
-// 1 KB (conflict-free).  A down block takes up to 4 row blocks of its tile with
-// one staging pipeline running across them.
+// Block: 256 weight rows x a tile of up to 16 NT tokens (NT columns of 16) of one group, 8
+// waves.  A wave owns two 16-row tiles (for gate_up the gate and the up rows of the same 16
+// outputs) and runs them against every column.  Per quad of 4 input groups it loads 64 bytes
+// of each of its rows straight into registers -- a lane the whole packed group kq of its row,
+// transposed within the lanes by permlane swaps -- expands each weight once for all the
+// tile's columns, and reads the columns' digits and factors from LDS, where the block stages
+// them in two buffers, a chunk of quads ahead.  The MFMA takes the digits as its A (rows:
+// tokens) and the weights as its B (columns: weight rows), so a lane's four results are of
+// one weight row, whose scale is a plain register, and of four tokens.  Loads of a quad are
+// issued a quad ahead, a step's two MFMAs one step (column, group, row tile) ahead of its
+// sums.  A group's tokens are split into equal tiles of whole columns (sw_mf_tile), and a
+// tile runs the loop of its own column count.
+//
+// What bounds it: the SIMDs' issue.  A step is 2 MFMAs, 4 conversions (one fma each), 4
+// products with s, 4 scalings (products or fmas with the power of two, exact) and 1-2 sums;
+// alone in registers, with two waves per SIMD, that takes 67 cycles -- MFMA and VALU time
+// add up -- against 130-160 here with the expansion (9 operations per 8 weights), LDS and
+// barriers.  LDS reads are 1 KB per step for two row tiles.  16 tokens (NT = 1) fit 128
+// registers, four waves per SIMD; 64 take 256, two.  Expanding in every wave from registers
+// replaced weights expanded once per block into LDS, whose reads (1 KB per row tile and
+// group) and barriers (one per chunk over 16 waves) bounded the loop: C2 S = 2048 gate_up
+// 1,676 -> 1,440 us, down 901 -> 776; S = 181 586 -> 447 and 320 -> 272.
 #include "sw_hip.h"
 #include "sw_gate.h"
 
 #define MF_DW 32           // digit dwords per (input row, group)
-#define MF_ROWS 128        // weight rows per block
-#define MF_TT SW_MF_TT     // tokens per block tile (64)
-#define MF_NT 1024         // threads per block: 16 waves, four per SIMD
-#define MF_CG 4            // input groups per staged chunk
-// the two chunk buffers in LDS, each operand's pair side by side (so that one base
-// register per operand and immediate offsets reach both): expanded weights
-// [buf][g][tile 8][quarter 4][row 16] x 16 B, digits [buf][g][token tile 4][op 2]
-// [quarter 4][token 16] x 16 B, scales [buf][g][row], token factors [buf][g][token]
-#define MF_A_SZ (MF_CG * MF_ROWS * 64)
-#define MF_B_SZ (MF_CG * MF_TT * 128)
-#define MF_S_SZ (MF_CG * MF_ROWS * 4)
-#define MF_X_SZ (MF_CG * MF_TT * 4)
-#define MF_A_OFF 0
-#define MF_B_OFF (MF_A_OFF + 2 * MF_A_SZ)
-#define MF_S_OFF (MF_B_OFF + 2 * MF_B_SZ)
-#define MF_X_OFF (MF_S_OFF + 2 * MF_S_SZ)
-#define MF_LDS_STAGE (MF_X_OFF + 2 * MF_X_SZ)
-#ifndef MF_PF
-#define MF_PF 1            // the next group's operands fetched during this group's products
-#endif
-#define MF_YLD 129         // floats per token row of a row block's gate and up sums (<= 32 tokens)
-#define MF_HLD 65          // floats per token row of h in the gate_up epilogue
-#define MF_EP_OFF MF_LDS_STAGE                            // the epilogue's own LDS
-#define MF_EP_SZ (MF_TT * MF_HLD * 4 > 32 * MF_YLD * 4 ? MF_TT * MF_HLD * 4 : 32 * MF_YLD * 4)
+#define MF_ROWS 256        // weight rows per block: 32 per wave
+#define MF_NTH 512         // threads per block: 8 waves
+// the (column, group) pairs of a staged chunk: 4 groups of up to four token columns, 8 of
+// two, or 8 of one (fewer staging registers where a wave has 128)
+#define MF_PAIRS(NT) ((NT) == 1 ? 8 : 16)
+// the two chunk buffers in LDS: digits [g][column][op 2][quarter 4][token 16] x 16 B, and
+// token factors [g][column][token]
+#define MF_B_SZ(NT) (MF_PAIRS(NT) * 2048)
+#define MF_X_SZ(NT) (MF_PAIRS(NT) * 64)
+#define MF_X_OFF(NT) (2 * MF_B_SZ(NT))
+#define MF_HLD 129         // floats per token row of h in the gate_up epilogue (64 rows within the buffers)
+
+template <int N>
+struct MfIc { static constexpr int v = N; };
 
 // ------------------------------------------------------------ digits ----
 // one group by the 32 lanes of a half-wave (i = lane in the half): the same
@@ -90,12 +84,11 @@ __device__ __forceinline__ void digits_group(float v, int i, uint32_t *__restric
     const float sc = (i & 1) ? 0.0625f : 1.0f;
     const uint32_t h0 = __builtin_bit_cast(uint16_t, (_Float16)((float)E0 * sc));
     const uint32_t h1 = __builtin_bit_cast(uint16_t, (_Float16)((float)E1 * sc));
-    // input r = i & 7 of quarter q = i >> 3 sits at f16 slot (r & 1) * 4 + (r >> 1) of the
-    // quarter's 4 dwords: inputs r and r ^ 2 share a dword (r & 2 the high half)
-    const uint32_t o0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h0, 0x4E, 0xF, 0xF, true);   // lane i ^ 2
-    const uint32_t o1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h1, 0x4E, 0xF, 0xF, true);
-    if ((i & 2) == 0) {
-        const int dw = (i >> 3) * 4 + (i & 1) * 2 + ((i >> 2) & 1);
+    // dword d of quarter q = i >> 3 holds inputs d (low half) and d + 4 (mf_expand's order)
+    const uint32_t o0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h0, 0x104, 0xF, 0xF, true);   // row_shl 4: lane i + 4
+    const uint32_t o1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h1, 0x104, 0xF, 0xF, true);
+    if ((i & 4) == 0) {
+        const int dw = (i >> 3) * 4 + (i & 3);
         dst[dw] = h0 | (o0 << 16);
         dst[16 + dw] = h1 | (o1 << 16);
     }
@@ -126,7 +119,7 @@ struct MfArgs {
     const uint32_t *dg;     // input digits [rows][G][MF_DW]
     const float *xs;        // input factors [rows][G]
     int dg_rows;            // rows of dg and xs (dg_rows * K * 4 < 2^32)
-    SwGroups grp;           // tiles: items of up to MF_TT tokens, P live
+    SwGroups grp;           // tiles: items of up to 16 NT tokens, P live
     int I;                  // GLU: the intermediate size (W.O == 2 I)
     int nrb;                // row blocks
     int rbper;              // row blocks per block (dividing nrb)
@@ -136,28 +129,36 @@ struct MfArgs {
     const SwTab *tab;       // per-group tensors (the _tab launches) or null
 };
 
-// the A operand of packed weight dword w (nibble n_r = w_r + 8 of input r of the
-// quarter at bits 4r) as f16 in the slot order of digits_group: (w0, w2), (w4, w6),
-// (16 w1, 16 w3), (16 w5, 16 w7).  An even input's nibble is the low nibble of a
-// byte, ORed under 0x64 into the f16 1024 + n; an odd input's is the high nibble,
-// giving 1024 + 16 n.  Adding -1032, resp. -1152, leaves w, resp. 16 w, exactly.
-__device__ __forceinline__ sw_i32x4 mf_expand(uint32_t w) {
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = w & 0xF0F0F0F0u, magic = 0x64646464u;
+// the weight operand of packed dword w (nibble n_r = w_r + 8 of input r of the quarter at
+// bits 4r) as f16 pairs (w0, w4), (16 w1, 16 w5), (w2, w6), (16 w3, 16 w7), the order of
+// digits_group.  Nibbles r and r + 4 sit 16 bits apart: masked out in place and ORed into
+// the mantissas of the f16 pair (1024, 1024) they give 1024 + n (bits 0-3) or 1024 + 16 n
+// (bits 4-7); adding -1032, resp. -1152, leaves w, resp. 16 w, exactly.  9 operations per
+// 8 weights, 4 of them on the packed f16 unit (which, like byte permutes and DPP, issues at
+// about 4.6 cycles against 2.7 for plain 32-bit operations, two or more waves per SIMD)
+__device__ __forceinline__ sw_half8 mf_expand(uint32_t w) {
+    const uint32_t lo = 0x000F000Fu, hi = 0x00F000F0u, magic = 0x64006400u, v = w >> 8;
     const sw_half2 off_lo = {(_Float16)-1032.0f, (_Float16)-1032.0f};
     const sw_half2 off_hi = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    // bytes (b0, 0x64, b1, 0x64) and (b2, 0x64, b3, 0x64) of lo and of hi
-    const uint32_t p0 = __builtin_amdgcn_perm(magic, lo, 0x04010400u), p1 = __builtin_amdgcn_perm(magic, lo, 0x04030402u);
-    const uint32_t p2 = __builtin_amdgcn_perm(magic, hi, 0x04010400u), p3 = __builtin_amdgcn_perm(magic, hi, 0x04030402u);
     sw_i32x4 a;
-    a[0] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, p0) + off_lo);
-    a[1] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, p1) + off_lo);
-    a[2] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, p2) + off_hi);
-    a[3] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, p3) + off_hi);
-    return a;
+    a[0] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, (w & lo) | magic) + off_lo);
+    a[1] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, (w & hi) | magic) + off_hi);
+    a[2] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, (v & lo) | magic) + off_lo);
+    a[3] = __builtin_bit_cast(int, __builtin_bit_cast(sw_half2, (v & hi) | magic) + off_hi);
+    return __builtin_bit_cast(sw_half8, a);
 }
 
-template <int N>
-struct MfIc { static constexpr int v = N; };
+// A lane loads 16 bytes of its row: the whole packed group kq = lane / 16 of a quad.
+// An MFMA of group g wants dword kq of group g in lane quarter kq, the transpose of
+// the 4 x 4 (lane quarter, dword) block: two swaps of lane halves, two of 16-lane rows
+__device__ __forceinline__ void mf_transpose(const sw_u32x4 &r, uint32_t (&o)[4]) {
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    const u2 a = __builtin_amdgcn_permlane32_swap(r.x, r.z, false, false);
+    const u2 b = __builtin_amdgcn_permlane32_swap(r.y, r.w, false, false);
+    const u2 c = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false);
+    const u2 d = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+    o[0] = c.x; o[1] = c.y; o[2] = d.x; o[3] = d.y;
+}
 
 // the value of lane J of each lane's quad (DPP quad_perm [J, J, J, J])
 template <int J>
@@ -165,369 +166,369 @@ __device__ __forceinline__ float mf_quad_bcast(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x55 * J, 0xF, 0xF, true));
 }
 
-template <int GLU, int CH, int FULL, int PT>
-__global__ __launch_bounds__(MF_NT, 1) void k_mf(MfArgs A) {
-    static_assert(MF_NT == 1024 && MF_CG * MF_ROWS == 512 && MF_CG * MF_TT * 8 == 2 * MF_NT, "staging map");
+// NT: the tile's most 16-token columns; SM: the weight scales, 0 one per row (after the
+// sum), 1 one per 32 inputs, 2 one per 64, 3 one per 128 or more (one a quad)
+template <int GLU, int NT, int SM, int PT>
+__global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
+    constexpr int CG = MF_PAIRS(NT) / NT, QPC = CG / 4;    // groups and quads per staged chunk
+    constexpr int PV = MF_PAIRS(NT) / 4;                   // digit units per staging thread and chunk
+    constexpr int B_SZ = MF_B_SZ(NT), X_SZ = MF_X_SZ(NT), X_OFF = MF_X_OFF(NT);
+    constexpr int RPB = GLU ? MF_ROWS / 2 : MF_ROWS;       // output rows a row block moves on by
+    static_assert(MF_NTH == 512, "staging map");
     extern __shared__ __align__(16) uint8_t mf_lds[];
     const SwQ4 W = A.W;
     const SwGroups grp = A.grp;
     const int K = W.K, G = K / SW_RG, O = W.O;
-    const int NC = G / MF_CG;                              // staged chunks (G % 4 == 0)
-    const int NCV = (G + CH - 1) / CH * (CH / MF_CG);      // chunks of the padded runs
+    const int NC = G / 4;                                  // quads of 4 groups
+    const int NCH = (NC + QPC - 1) / QPC;                  // staged chunks of a row block
+    const int NQ = G > 8 ? 4 : NC;                         // quads per run (G = 4, 8: one short run)
     // (the wave index in a scalar register: what derives from it is uniform to the compiler)
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15,
               kq = lane >> 4;
 
-    // block -> (tile, row block), XCD-aware over the live blocks
-    // (a block takes rbper consecutive row blocks of one tile, its chunk pipeline running on
-    // from one row block to the next: one start and one drain per rbper row blocks)
-    const int rbper = GLU ? 1 : A.rbper;                   // (gate_up: one, known to the compiler)
-    const int nrg = A.nrb / rbper;                         // row-block runs per tile
+    // block -> (tile, run of rbper row blocks), XCD-aware over the live blocks; the chunk
+    // pipeline runs on from one row block to the next
+    const int rbper = GLU ? 1 : A.rbper;
+    const int nrg = A.nrb / rbper;
     const int nlive = *grp.P * nrg;
     if ((int)blockIdx.x >= nlive) return;
     const int wk = sw_xcd_work((int)blockIdx.x, nlive);
     const int tile = wk / nrg, rbf = (wk - tile * nrg) * rbper;     // the block's first row block
     int e, beg, t0, tend;
-    if (!grp_work(grp, tile, MF_TT, e, beg, t0, tend)) return;
-    const int nt = tend - t0, nact = (nt + 15) >> 4;       // tokens, token tiles with tokens
-    const int i0 = rbf * 64, r0 = rbf * MF_ROWS;           // (of the first row block)
-    constexpr int RPB = GLU ? 64 : MF_ROWS;                // weight rows a row block moves on by
-    // weight row of local row r (GLU: gate rows i0..i0+63, then the up rows)
-    // (PT: row r of the group's own gate, up or down tensor)
-    auto srow = [&](int r) -> uint32_t {
-        const uint32_t eo = PT ? 0u : (uint32_t)e * (uint32_t)O;
-        if (GLU) return eo + (uint32_t)(r < 64 ? i0 + r : (PT ? 0 : A.I) + i0 + r - 64);
-        return eo + (uint32_t)(r0 + r);     // past O: the next expert's rows (PT: zeros), not stored
-    };
-    auto token = [&](int t) -> int64_t {                   // input row of tile token t (past the tile: its last)
+    if (!grp_work(grp, tile, 16 * NT, e, beg, t0, tend)) return;
+    const int nt = tend - t0, nact = (nt + 15) >> 4;       // tokens, token columns with tokens
+    auto token = [&](int t) -> uint32_t {                  // input row of tile token t (past the tile: its last)
         const int pr = beg + t0 + min(t, nt - 1);
-        return grp.grow ? grp.grow[pr] : pr;
+        return (uint32_t)(grp.grow ? grp.grow[pr] : pr);
     };
     const int ng = W.gs > 0 ? K / W.gs : 1;
-    const uint32_t rbytes = (uint32_t)K / 2;
-    // staging roles by whole waves; for gate_up rotated so that in a tile of 1-3 token tiles the
-    // computing waves take the roles with no work (the digits of token tiles that do not
-    // compute are not staged) or the lightest
-    const int rot = GLU ? (nact == 1 ? 10 : nact < 4 ? 8 : 0) : 0;
-    const int st = (tid + 64 * rot) & (MF_NT - 1);
-    const int sw_ = __builtin_amdgcn_readfirstlane(st >> 6);   // the staging role's wave index
-    sw_rsrc rq, rs;
+    const uint32_t rbytes = (uint32_t)K / 2, sbytes = (uint32_t)ng * 4;
+    sw_rsrc rq[2], rs[2];                                  // row tile t's tensor
     if constexpr (PT) {
-        // a staging thread's row ra (below) is an up row iff (st >> 9) & 1: uniform per wave
         const SwTab tb_ = A.tab[e];
-        if (GLU) {
-            const bool up = (sw_ >> 3) & 1;
-            rq = sw_make_rsrc(up ? tb_.u : tb_.g, (uint32_t)A.I * rbytes);
-            rs = sw_make_rsrc(up ? tb_.us : tb_.gs, (uint32_t)A.I * (uint32_t)ng * 4);
-        } else {
-            rq = sw_make_rsrc(tb_.d, (uint32_t)O * rbytes);
-            rs = sw_make_rsrc(tb_.ds, (uint32_t)O * (uint32_t)ng * 4);
-        }
+        const uint32_t rows = (uint32_t)(GLU ? A.I : O);
+        rq[0] = sw_make_rsrc(GLU ? tb_.g : tb_.d, rows * rbytes);
+        rq[1] = sw_make_rsrc(GLU ? tb_.u : tb_.d, rows * rbytes);
+        rs[0] = sw_make_rsrc(GLU ? tb_.gs : tb_.ds, rows * sbytes);
+        rs[1] = sw_make_rsrc(GLU ? tb_.us : tb_.ds, rows * sbytes);
     } else {
-        rq = sw_q4_rq(W);
-        rs = sw_q4_rs(W);
+        rq[0] = rq[1] = sw_q4_rq(W);
+        rs[0] = rs[1] = sw_q4_rs(W);
     }
-
-    // ---- staging: the units of a chunk of staging slot st
-    //  weights (every slot): half hq of row ra's 16 B packed of group ga (below; expanded on
-    //           the store); slots of half 0 also the row's scale of the group
-    //  digits:  16 B (op, quarter) of token tb of groups st >> 9 and (st >> 9) + 2: unit u of a
-    //           group is token tile u >> 7, op (u >> 6) & 1, quarter (u >> 4) & 3, token u & 15;
-    //           staged only for the token tiles that compute (dact)
-    //  factors (the 4 waves with sw_ % 4 == 1): token tx of group gx (as ra, ga)
-    // (the staging work spread evenly over the 16 waves: the chunk's barrier waits for the
-    // slowest)
-    // Every load is a buffer load: the slot's part of its offset in a register set once,
-    // the chunk's in a scalar offset.
-    constexpr int DG_PER = MF_CG * MF_TT * 8 / MF_NT;      // digit units per slot (2)
-    // (a wave's 64 slots: one half of 16 rows, each with the chunk's 4 groups, side by side in
-    // memory -- a wave load touches 16 lines, not 64 -- the rows fastest within each 16-slot
-    // quarter, so that the LDS stores stay conflict-free)
-    const int ra = ((st >> 7) << 4) | (st & 15), ga = (st >> 4) & 3, hq = (st >> 6) & 1;
-    const bool sst = hq == 0;                              // uniform per wave
-    const uint32_t rowa = srow(ra);
-    const int tb = ((st >> 7) & 3) * 16 + (st & 15), opb = (st >> 6) & 1, kqb = (st >> 4) & 3, gb = st >> 9;
-    const int xi = ((sw_ >> 2) << 6) | (st & 63);         // (factor slot)
-    const int tx = ((xi >> 6) << 4) | (xi & 15), gx = (xi >> 4) & 3;   // (as ra, ga)
-    const bool dact = ((sw_ >> 1) & 3) < nact;            // uniform per wave
-    const bool xst = (sw_ & 3) == 1;
+    // ---- the wave's weight rows: row tile 0 and 1 start at tensor rows wr0, wr1.  gate_up:
+    // the gate and the up rows of the same 16 outputs; down: 32 rows in a line (a wave past
+    // O, where O is an odd number of half blocks, reads the last rows and stores nothing)
+    const int lr = (GLU ? 16 : 32) * wave;                 // the wave's rows in a row block
+    const uint32_t eo = PT ? 0u : (uint32_t)e * (uint32_t)O;
+    auto wrow = [&](int t, int rb) -> uint32_t {
+        if constexpr (GLU) return eo + (uint32_t)(rb * RPB + lr + (t && !PT ? A.I : 0));
+        return eo + (uint32_t)(min(rb * RPB + lr, O - 32) + 16 * t);
+    };
+    struct Raw { sw_u32x4 q[2]; sw_f32x4 s[2]; };
+    // quad c of row block rb: 64 bytes of each of the tile's 16 rows, and lane col & 3's
+    // scales of row 4 kq + (col & 3) (moved to the quad's products by DPP)
+    auto load_w = [&](Raw &R, int rb, int c) {
+        const uint32_t cu = (uint32_t)__builtin_amdgcn_readfirstlane(c);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint32_t r0 = wrow(t, rb);
+            R.q[t] = sw_ld16(rq[t], (r0 + (uint32_t)col) * rbytes + (uint32_t)kq * 16, cu * 64);
+            const uint32_t vs = (r0 + (uint32_t)col) * sbytes;
+            if constexpr (SM == 1) R.s[t] = __builtin_bit_cast(sw_f32x4, sw_ld16(rs[t], vs, cu * 16));
+            if constexpr (SM == 2) {
+                const uint2 v = sw_ld8(rs[t], vs, cu * 8);
+                R.s[t][0] = R.s[t][1] = __builtin_bit_cast(float, v.x);
+                R.s[t][2] = R.s[t][3] = __builtin_bit_cast(float, v.y);
+            }
+            if constexpr (SM == 3) {
+                const float v = sw_ld4f(rs[t], vs, ((cu * 128) >> A.gsh) * 4);
+                R.s[t] = sw_f32x4{v, v, v, v};
+            }
+        }
+    };
+    // ---- staging a chunk of CG groups: the digits in 16-byte units [g][column][op][quarter]
+    // [token], PV per thread (unit v * 512 + tid: one wave load is 64 bytes of 16 tokens, one
+    // wave store 1 KB in a line), and the token factors [g][column][token], one each by the
+    // first threads.  Columns with no tokens are not staged.
+    const int dtok = tid & 15, dpart = ((tid >> 6) & 1) * 64 + ((tid >> 4) & 3) * 16, drc = tid >> 7;
+    const int dcol = __builtin_amdgcn_readfirstlane(drc % NT), dg0 = drc / NT;      // uniform per wave
+    const int xg = NT == 1 ? (tid >> 4) & 7 : ((tid >> 4) & 3) + (NT == 2 ? 4 * ((tid >> 6) & 1) : 0);
+    const int xcol = __builtin_amdgcn_readfirstlane(NT == 1 ? 0 : NT == 2 ? (tid >> 7) & 1 : (tid >> 6) & 3);
+    const bool dact = dcol < nact, xact = wave < MF_PAIRS(NT) / 4 && xcol < nact;
     const sw_rsrc rd = sw_make_rsrc(A.dg, (uint32_t)A.dg_rows * (uint32_t)G * MF_DW * 4);
     const sw_rsrc rx = sw_make_rsrc(A.xs, (uint32_t)A.dg_rows * (uint32_t)G * 4);
-    const uint32_t vq = rowa * rbytes + (uint32_t)ga * 16 + (uint32_t)hq * 8;
-    const uint32_t vs = (rowa * (uint32_t)ng + (uint32_t)((ga * SW_RG) >> A.gsh)) * 4;
-    const uint32_t vd = ((uint32_t)token(tb) * (uint32_t)G + (uint32_t)gb) * MF_DW * 4 + (uint32_t)(opb * 16 + kqb * 4) * 4;
-    const uint32_t vx = ((uint32_t)token(tx) * (uint32_t)G + (uint32_t)gx) * 4;
-    uint2 pka;
-    sw_u32x4 pkb[DG_PER];
-    float psa = 1.0f, pxf = 0.f;
-    // chunk q of the block: chunk q % NCV of its row block q / NCV (the row block's rows in
-    // the vector offset, which the range check covers)
-    auto stage_load = [&](int q) {
-        const int rbi = GLU ? 0 : q / NCV, c = q - rbi * NCV;
-        const uint32_t g0 = (uint32_t)__builtin_amdgcn_readfirstlane(c * MF_CG);
-        const uint32_t dr = (uint32_t)(rbi * RPB);
-        pka = sw_ld8(rq, vq + dr * rbytes, g0 * 16);
-        // ((g0 + ga) * 32) >> gsh splits: g0 * 32 is a multiple of 128, ga * 32 < 128
-        if (sst && W.gs > 0) psa = sw_ld4f(rs, vs + dr * (uint32_t)ng * 4, ((g0 * SW_RG) >> A.gsh) * 4);
-        if (dact)
+    // (every load is unconditional -- an empty column's of column 0, from cache -- so that the
+    // compiler's wait counts stay exact; only the stores are skipped)
+    const uint32_t vd = token(16 * (dact ? dcol : 0) + dtok) * (uint32_t)G * (MF_DW * 4) + (uint32_t)dpart;
+    const uint32_t vx = token(16 * (xcol < nact ? xcol : 0) + dtok) * (uint32_t)G * 4;
+    sw_u32x4 pkb[PV];
+    float pxf = 0.f;
+    auto stage_load = [&](int ch) {                        // chunk ch % NCH of a row block (groups past G: the last)
+        const int g0 = __builtin_amdgcn_readfirstlane((GLU ? ch : ch % NCH) * CG);
+        if constexpr (QPC == 1) {                          // (never past G)
 #pragma unroll
-            for (int v = 0; v < DG_PER; v++) pkb[v] = sw_ld16(rd, vd + (uint32_t)v * 2 * MF_DW * 4, g0 * MF_DW * 4);
-        if (xst) pxf = sw_ld4f(rx, vx, g0 * 4);
+            for (int v = 0; v < PV; v++) pkb[v] = sw_ld16(rd, vd, (uint32_t)(g0 + v) * (MF_DW * 4));
+            pxf = sw_ld4f(rx, vx + (uint32_t)xg * 4, (uint32_t)g0 * 4);
+        } else {
+#pragma unroll
+            for (int v = 0; v < PV; v++) pkb[v] = sw_ld16(rd, vd + (uint32_t)min(g0 + dg0 + v * (4 / NT), G - 1) * (MF_DW * 4), 0);
+            pxf = sw_ld4f(rx, vx + (uint32_t)min(g0 + xg, G - 1) * 4, 0);
+        }
     };
     auto stage_store = [&](int buf) {
-        sw_i32x4 *Al = (sw_i32x4 *)(mf_lds + MF_A_OFF + buf * MF_A_SZ);
-        sw_u32x4 *Bl = (sw_u32x4 *)(mf_lds + MF_B_OFF + buf * MF_B_SZ);
-        {
-            const int m = ra >> 4, i = ra & 15;
-            Al[((ga * 8 + m) * 4 + 2 * hq) * 16 + i] = mf_expand(pka.x);
-            Al[((ga * 8 + m) * 4 + 2 * hq + 1) * 16 + i] = mf_expand(pka.y);
-            if (sst) ((float *)(mf_lds + MF_S_OFF + buf * MF_S_SZ))[ga * MF_ROWS + ra] = psa;
-        }
+        sw_u32x4 *Bl = (sw_u32x4 *)(mf_lds + buf * B_SZ);
         if (dact)
 #pragma unroll
-            for (int v = 0; v < DG_PER; v++) Bl[v * MF_NT + st] = pkb[v];
-        if (xst) ((float *)(mf_lds + MF_X_OFF + buf * MF_X_SZ))[gx * MF_TT + tx] = pxf;
+            for (int v = 0; v < PV; v++) Bl[v * MF_NTH + tid] = pkb[v];
+        if (xact) ((float *)(mf_lds + X_OFF + buf * X_SZ))[(xg * NT + xcol) * 16 + dtok] = pxf;
     };
 
-    // ---- the compute waves' (row tile, token tile) pairs: two per wave (row tiles m, m + 4
-    // of token tile w >> 2) when 3-4 token tiles compute, else one (row tile w & 7 of token
-    // tile w >> 3), so that a tail tile's pairs still spread over all four SIMDs, two or
-    // four waves on each
-    constexpr int NQ = CH / MF_CG;                         // chunks per run
-    const int NR = NCV / NQ;                               // runs
-    // the terms of one chunk's 4 groups summed as ((p0 + p1) + (p2 + p3)) per (row, token)
-    // into q (REAL = 0: the +0 terms of a run's padding, whose sum is +0)
-    auto quad = [&](auto NPC, auto RC, int buf, int tt, int m0, sw_f32x4 (&q)[2]) {
-        constexpr int NP = decltype(NPC)::v;
-        if constexpr (!decltype(RC)::v) {
-#pragma unroll
-            for (int mi = 0; mi < NP; mi++) q[mi] = sw_f32x4{0.f, 0.f, 0.f, 0.f};
-            return;
-        } else {
-            // this lane's operands of group g: one base per operand plus immediate offsets
-            const uint8_t *pa = mf_lds + MF_A_OFF + buf * MF_A_SZ + ((m0 * 4 + kq) * 16 + col) * 16;
-            const uint8_t *pb = mf_lds + MF_B_OFF + buf * MF_B_SZ + (tt * 2 * 64 + lane) * 16;
-            const uint8_t *ps = mf_lds + MF_S_OFF + buf * MF_S_SZ + (16 * m0 + 4 * kq) * 4;
-            const uint8_t *px = mf_lds + MF_X_OFF + buf * MF_X_SZ + (16 * tt + col) * 4;
-            sw_f32x4 h[NP];                                // the pending pair (p0 + p1)
-            // a lane's four rows 4 kq + j take their scales from the four lanes of its quad
-            // (lane col & 3 reads row 4 kq + (col & 3)), moved by DPP into the products: a
-            // quarter of the LDS reads of one 16-byte read per lane
-            struct Frag {
-                sw_half8 a[NP], b0, b1;
-                float s1[NP];
-                float xf;
-            };
-            auto fetch = [&](Frag &F, int g) {
-#pragma unroll
-                for (int mi = 0; mi < NP; mi++) {
-                    F.a[mi] = *(const sw_half8 *)(pa + (g * 8 + 4 * mi) * 4 * 16 * 16);
-                    F.s1[mi] = *(const float *)(ps + (g * MF_ROWS + 64 * mi + (col & 3)) * 4);
-                }
-                F.b0 = *(const sw_half8 *)(pb + (g * 4 * 2 + 0) * 64 * 16);
-                F.b1 = *(const sw_half8 *)(pb + (g * 4 * 2 + 1) * 64 * 16);
-                F.xf = *(const float *)(px + g * MF_TT * 4);
-            };
-            Frag Fr[2];
-            if (MF_PF) fetch(Fr[0], 0);
-#pragma unroll
-            for (int g = 0; g < MF_CG; g++) {
-                if (!MF_PF) fetch(Fr[g & 1], g);
-                const Frag &C = Fr[g & 1];
-                const sw_f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                sw_f32x4 R0[NP], R1[NP];
-                // the MFMAs issue at raised wave priority: the SIMD's waves, which leave each
-                // chunk's barrier together, then spread out instead of waiting on their
-                // products in step
-                __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-                for (int mi = 0; mi < NP; mi++) {
-                    R0[mi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(C.a[mi], C.b0, z, 0, 0, 0);
-                    R1[mi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(C.a[mi], C.b1, z, 0, 0, 0);
-                }
-                __builtin_amdgcn_s_setprio(0);
-                // (MF_PF: the next group's operands load while these products finish)
-                if (MF_PF && g + 1 < MF_CG) fetch(Fr[(g + 1) & 1], g + 1);
-#pragma unroll
-                for (int mi = 0; mi < NP; mi++) {
-                    // s * 2^(e - 21) of rows 4 kq + j (the DPP moves fold into the products)
-                    const float t4[4] = {mf_quad_bcast<0>(C.s1[mi]) * C.xf, mf_quad_bcast<1>(C.s1[mi]) * C.xf,
-                                         mf_quad_bcast<2>(C.s1[mi]) * C.xf, mf_quad_bcast<3>(C.s1[mi]) * C.xf};
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        // (float)acc exactly, times (s * 2^(e - 21)), as dot8's term
-                        const float p = __builtin_fmaf(R1[mi][j], 4096.0f, R0[mi][j]) * t4[j];
-                        if (g == 0 || g == 2) h[mi][j] = p;
-                        else if (g == 1) q[mi][j] = h[mi][j] + p;
-                        else q[mi][j] = q[mi][j] + (h[mi][j] + p);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);         // one group's operands in flight at a time
-            }
-        }
-    };
-    // a row block's sums out: gate_up, h = silu(gate) * up to its digits (two limb
+    // a row block's sums out: gate_up, h = silu(gate) * up through LDS to its digits (four
     // groups of the down's input per token); down, the rows of each token
-    auto epilogue = [&](auto NPC, int rb, const sw_f32x4 (&y)[2], int tt, int m0, bool wact) {
-        constexpr int NP = decltype(NPC)::v;
-        const int ib = rb * 64, rr0 = rb * MF_ROWS;
+    auto epilogue = [&](auto NAC, int rb, const sw_f32x4 (&y)[2][decltype(NAC)::v]) {
+        constexpr int NA = decltype(NAC)::v;
         if constexpr (GLU) {
-            const int I = A.I;
-            float *el = (float *)(mf_lds + MF_EP_OFF);
-            auto gsc = [&](int i) -> float { return PT ? A.tab[e].gs[ib + i] : W.s[(int64_t)e * (2 * I) + ib + i]; };
-            auto usc = [&](int i) -> float { return PT ? A.tab[e].us[ib + i] : W.s[(int64_t)e * (2 * I) + I + ib + i]; };
-            if constexpr (NP == 2) {
-                // a lane holds the gate (row tile m0) and up (m0 + 4) sums of outputs 16 m0 + 4 kq + j
-                if (wact)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int i = 16 * m0 + 4 * kq + j, t = 16 * tt + col;
-                        float yg = y[0][j], yu = y[1][j];
-                        if (W.gs <= 0) {                        // per-row scales after the sum
-                            yg = yg * gsc(i);
-                            yu = yu * usc(i);
-                        }
-                        el[t * MF_HLD + i] = (yg / (1.0f + expf(-yg))) * yu;
-                    }
-            } else {
-                // (one row tile per wave: the gate and up sums of at most 32 tokens as they are)
-                if (wact)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) el[(16 * tt + col) * MF_YLD + 16 * m0 + 4 * kq + j] = y[0][j];
+            const int I = A.I, ib = rb * RPB;
+            float *el = (float *)mf_lds;                   // (the chunk buffers: every wave is past its last read)
+            const int i = lr + col;                        // the lane's output, of tokens 4 kq .. + 3
+            float gsc = 1.f, usc = 1.f;
+            if constexpr (SM == 0) {                       // per-row scales after the sum
+                gsc = PT ? A.tab[e].gs[ib + i] : W.s[(int64_t)e * O + ib + i];
+                usc = PT ? A.tab[e].us[ib + i] : W.s[(int64_t)e * O + I + ib + i];
             }
-            __syncthreads();
-            // the row block's 64 outputs are two limb groups of the down projection's input
-            const int GI = I / SW_RG, hw = tid >> 5, i = tid & 31;
-            for (int job = hw; job < 2 * nt; job += MF_NT / 32) {
-                const int t = job >> 1, q = job & 1;
-                const int64_t prow = beg + t0 + t;
-                const int gi = 2 * rb + q;
-                float h;
-                if constexpr (NP == 2) {
-                    h = el[t * MF_HLD + 32 * q + i];
-                } else {
-                    const int o = 32 * q + i;
-                    float yg = el[t * MF_YLD + o], yu = el[t * MF_YLD + 64 + o];
-                    if (W.gs <= 0) {
-                        yg = yg * gsc(o);
-                        yu = yu * usc(o);
+#pragma unroll
+            for (int c = 0; c < NA; c++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    float yg = y[0][c][j], yu = y[1][c][j];
+                    if constexpr (SM == 0) {
+                        yg = yg * gsc;
+                        yu = yu * usc;
                     }
-                    h = (yg / (1.0f + expf(-yg))) * yu;
+                    el[(16 * c + 4 * kq + j) * MF_HLD + i] = (yg / (1.0f + expf(-yg))) * yu;
                 }
-                digits_group(h, i, A.hdg + (prow * GI + gi) * MF_DW, A.hxs + prow * GI + gi);
+            __syncthreads();
+            const int GI = I / SW_RG, hw = tid >> 5, ih = tid & 31;
+            for (int job = hw; job < 4 * nt; job += MF_NTH / 32) {
+                const int t = job >> 2, q = job & 3, gi = ib / SW_RG + q;
+                const int64_t prow = beg + t0 + t;
+                digits_group(el[t * MF_HLD + 32 * q + ih], ih, A.hdg + (prow * GI + gi) * MF_DW, A.hxs + prow * GI + gi);
             }
         } else {
-            // a lane holds rows 16 m + 4 kq .. + 3 of token 16 tt + col: one 16-byte store each
-            const int t = 16 * tt + col;
-            if (wact && t < nt) {
-                float *yrow = A.Y + (int64_t)(beg + t0 + t) * O;
+            const int row0 = rb * RPB + lr;
+            if (row0 >= O) return;                         // uniform per wave
 #pragma unroll
-                for (int mi = 0; mi < NP; mi++) {
-                    const int row = rr0 + 16 * (m0 + 4 * mi) + 4 * kq;
-                    if (row < O) {
-                        sw_f32x4 o;
+            for (int rt = 0; rt < 2; rt++) {
+                const int row = row0 + 16 * rt + col;      // the lane's row, of tokens 4 kq .. + 3
+                const float ds = SM ? 1.f : PT ? A.tab[e].ds[row] : W.s[(int64_t)e * O + row];
 #pragma unroll
-                        for (int j = 0; j < 4; j++)
-                            o[j] = W.gs > 0 ? y[mi][j] : y[mi][j] * (PT ? A.tab[e].ds[row + j] : W.s[(int64_t)e * O + row + j]);
-                        *(sw_f32x4 *)(yrow + row) = o;
+                for (int c = 0; c < NA; c++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const int t = 16 * c + 4 * kq + j;
+                        if (t < nt) A.Y[(int64_t)(beg + t0 + t) * O + row] = SM ? y[rt][c][j] : y[rt][c][j] * ds;
                     }
-                }
             }
-        }
-    };
-    // the main loop for NP pairs per wave: for each of the block's row blocks, runs of NQ
-    // chunks, each run's quads summed ((q0 + q1) + (q2 + q3)) (NQ = 4), the runs added
-    // left to right into y; then the row block's epilogue.  The staging runs over the
-    // block's chunks q = rbi NCV + c without a break between row blocks.
-    const int QT = rbper * NCV;
-    auto real = [&](int q) { return GLU ? q < NC : q - q / NCV * NCV < NC; };
-    auto main_loop = [&](auto NPC) {
-        constexpr int NP = decltype(NPC)::v;
-        const int tt = NP == 2 ? wave >> 2 : wave >> 3, m0 = NP == 2 ? wave & 3 : wave & 7;
-        const bool wact = tt < nact;                       // uniform over the wave
-        for (int rbi = 0; rbi < rbper; rbi++) {
-            sw_f32x4 y[2];
-            for (int r = 0; r < NR; r++) {
-                sw_f32x4 ra[NP], rb[NP], q[2];
-#pragma unroll
-                for (int Q = 0; Q < NQ; Q++) {
-                    const int c = r * NQ + Q, qg = rbi * NCV + c;
-                    const int buf = NQ > 1 ? (Q & 1) : (qg & 1);   // (NCV is even when NQ > 1)
-                    if (wact) {
-                        // (a run-time test also for FULL: as a branch it keeps the compiler from
-                        // interleaving the unrolled chunks, which spills at 128 registers)
-                        if (c < NC) quad(NPC, MfIc<1>{}, buf, tt, m0, q);
-                        else quad(NPC, MfIc<0>{}, buf, tt, m0, q);
-#pragma unroll
-                        for (int mi = 0; mi < NP; mi++) {
-                            if (Q == 0) ra[mi] = q[mi];
-                            else if (Q == 1 && NQ == 4) ra[mi] = ra[mi] + q[mi];
-                            else if (Q == 2) rb[mi] = q[mi];
-                            else if (Q == 3) ra[mi] = ra[mi] + (rb[mi] + q[mi]);
-                            else ra[mi] = ra[mi] + q[mi];  // Q == 1 of NQ == 2
-                        }
-                    }
-                    if (qg + 1 < QT && real(qg + 1)) stage_store((qg + 1) & 1);  // read by no wave since the last barrier
-                    if (qg + 2 < QT && real(qg + 2)) stage_load(qg + 2);         // registers only: issued before the barrier's wait
-                    __syncthreads();
-                }
-                if (wact)
-#pragma unroll
-                    for (int mi = 0; mi < NP; mi++) y[mi] = r == 0 ? ra[mi] : y[mi] + ra[mi];
-            }
-            epilogue(NPC, rbf + rbi, y, tt, m0, wact);
         }
     };
 
-    stage_load(0);
-    stage_store(0);
-    if (QT > 1 && real(1)) stage_load(1);
-    __syncthreads();
-    if (nact > 2) main_loop(MfIc<2>{});
-    else main_loop(MfIc<1>{});
+    auto main_loop = [&](auto NAC) {
+        constexpr int NA = decltype(NAC)::v;               // the tile's token columns
+        Raw raw;
+        load_w(raw, rbf, 0);
+        stage_load(0);
+        stage_store(0);
+        const int QT = rbper * NCH;                        // the block's chunks
+        stage_load(min(1, QT - 1));
+        int ch = 0;                                        // the chunk in LDS buffer ch & 1
+        __syncthreads();
+        // quad qc of row block rb into acc.  All loads -- the next quad's weights, the next
+        // chunk's digits -- are issued at its top and waited for at the next one's or at the
+        // chunk's end, a whole quad's work later: issued at its end, the next top's wait for
+        // the (older) weights would drain them too
+        auto quad = [&](int rb, int qc, sw_f32x4 (&acc)[2][NA]) {
+            // the quad's operands: 4 groups of both row tiles, then the next quad's loads
+            // (expanded once for several columns; for a single one group by group, in registers)
+            sw_half8 a[2][NA > 1 ? 4 : 1];
+            uint32_t w[2][4];
+            sw_f32x4 sc[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                mf_transpose(raw.q[t], w[t]);
+                if constexpr (NA > 1)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) a[t][g] = mf_expand(w[t][g]);
+                if constexpr (SM) sc[t] = raw.s[t];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            {
+                const bool more = qc + 1 < NC;
+                load_w(raw, more ? rb : min(rb + 1, rbf + rbper - 1), more ? qc + 1 : 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const int gl = qc % QPC * 4;               // the quad's first group in its chunk
+            const uint8_t *pb = mf_lds + (ch & 1) * B_SZ + gl * NT * 2048 + lane * 16;
+            const uint8_t *px = mf_lds + X_OFF + (ch & 1) * X_SZ + (gl * NT * 16 + 4 * kq) * 4;
+            // steps (column c, group g, row tile t), t fastest: a (c, g)'s digits are read two
+            // (c, g) ahead, a step's two MFMAs issued one step ahead of its sums
+            struct Op { sw_half8 b0, b1; sw_f32x4 xf; } op[2];
+            sw_f32x4 R[2][2];
+            auto fetch = [&](int k, Op &o) {
+                const int c = k >> 2, g = k & 3;
+                o.b0 = *(const sw_half8 *)(pb + (g * NT + c) * 2048);
+                o.b1 = *(const sw_half8 *)(pb + (g * NT + c) * 2048 + 1024);
+                o.xf = *(const sw_f32x4 *)(px + (g * NT + c) * 64);
+            };
+            auto mul = [&](int i, const Op &o, sw_f32x4 (&r_)[2]) {
+                const sw_f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                const int t = i & 1, g = (i >> 1) & 3;
+                const sw_half8 av = NA > 1 ? a[t][NA > 1 ? g : 0] : mf_expand(w[t][g]);
+                r_[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.b0, av, z, 0, 0, 0);
+                r_[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.b1, av, z, 0, 0, 0);
+            };
+            constexpr int NS = 8 * NA;
+            fetch(0, op[0]);
+            fetch(1, op[1]);
+            mul(0, op[0], R[0]);
+            sw_f32x4 h[2], q[2];
+#pragma unroll
+            for (int i = 0; i < NS; i++) {
+                const int c = i >> 3, g = (i >> 1) & 3, t = i & 1;
+                const sw_f32x4 xf = op[(i >> 1) & 1].xf;
+                if (i + 1 < NS) mul(i + 1, op[((i + 1) >> 1) & 1], R[(i + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                // (float)acc exactly, times s, times the token's power of two: dot8's
+                // (float)acc * (s * xf) with its one rounding, the second of a pair scaled by
+                // the fma that adds it
+                sw_f32x4 u;
+#pragma unroll
+                for (int j = 0; j < 4; j++) u[j] = __builtin_fmaf(R[i & 1][1][j], 4096.0f, R[i & 1][0][j]);
+                if constexpr (SM) u = u * sc[t][g];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (g == 0 || g == 2) h[t][j] = u[j] * xf[j];
+                    else if (g == 1) q[t][j] = __builtin_fmaf(u[j], xf[j], h[t][j]);
+                    else q[t][j] = q[t][j] + __builtin_fmaf(u[j], xf[j], h[t][j]);
+                }
+                // (formed here: the compiler would sink the sums to their last use, with every
+                // product live until then)
+                if (g == 0 || g == 2) asm volatile("" : "+v"(h[t]));
+                else asm volatile("" : "+v"(q[t]));
+                if (t == 1 && (i >> 1) + 2 < NS / 2) fetch((i >> 1) + 2, op[(i >> 1) & 1]);
+                if (g == 3) acc[t][c] = acc[t][c] + q[t];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the chunk's last quad: the next chunk into the other buffer (read by no wave since
+            // the last barrier)
+            if (qc % QPC == QPC - 1 || qc == NC - 1) {
+                if (ch + 1 < QT) stage_store((ch + 1) & 1);
+                stage_load(min(ch + 2, QT - 1));
+                ch++;
+                __syncthreads();
+            }
+        };
+        auto fill = [&](sw_f32x4 (&v)[2][NA], float x) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int c = 0; c < NA; c++) v[t][c] = sw_f32x4{x, x, x, x};
+        };
+        // (sums start from -0, the identity of f32 addition: the first term's bits as they are)
+        for (int rbi = 0; rbi < rbper; rbi++) {
+            const int rb = rbf + rbi;
+            sw_f32x4 y[2][NA];
+            fill(y, -0.f);
+#pragma unroll 1
+            for (int r0 = 0; r0 < NC; r0 += 4) {
+                // a run: (q0 + q1) + (q2 + q3), a short last run padded with +0 terms
+                sw_f32x4 ra[2][NA], rv[2][NA];
+                fill(ra, -0.f);
+#pragma unroll 1
+                for (int qc = r0; qc < min(r0 + 2, NC); qc++) quad(rb, qc, ra);
+                if (NQ == 4) {
+                    fill(rv, r0 + 2 < NC ? -0.f : 0.f);
+#pragma unroll 1
+                    for (int qc = r0 + 2; qc < min(r0 + 4, NC); qc++) quad(rb, qc, rv);
+                    if (r0 + 4 > NC) {
+#pragma unroll
+                        for (int t = 0; t < 2; t++)
+#pragma unroll
+                            for (int c = 0; c < NA; c++) {
+                                if (r0 + 1 == NC) ra[t][c] = ra[t][c] + 0.f;
+                                rv[t][c] = rv[t][c] + 0.f;
+                            }
+                    }
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int c = 0; c < NA; c++) ra[t][c] = ra[t][c] + rv[t][c];
+                }
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int c = 0; c < NA; c++) y[t][c] = y[t][c] + ra[t][c];
+            }
+            epilogue(NAC, rb, y);
+        }
+    };
+    if constexpr (NT == 1) main_loop(MfIc<1>{});
+    else if constexpr (NT == 2) {
+        if (nact == 1) main_loop(MfIc<1>{});
+        else main_loop(MfIc<2>{});
+    } else {
+        if (nact == 1) main_loop(MfIc<1>{});
+        else if (nact == 2) main_loop(MfIc<2>{});
+        else if (nact == 3) main_loop(MfIc<3>{});
+        else main_loop(MfIc<4>{});
+    }
 }
 
 // ------------------------------------------------------------ launch ----
-static size_t mf_lds_bytes() { return (size_t)MF_EP_OFF + MF_EP_SZ; }
+// the chunk buffers; the gate_up epilogue's h lies over them
+template <int NT>
+static size_t mf_lds_bytes() {
+    const size_t b = MF_X_OFF(NT) + 2 * MF_X_SZ(NT), h = (size_t)16 * NT * MF_HLD * 4;
+    return b > h ? b : h;
+}
 // dynamic LDS above 64 KB, raised once per kernel, outside any stream work
-template <int GLU, int CH, int FULL, int PT>
+template <int GLU, int NT, int SM, int PT>
 static int mf_go(hipStream_t st, unsigned nblocks, const MfArgs &A) {
     static size_t raised = 0;
-    const size_t lds = mf_lds_bytes();
+    const size_t lds = mf_lds_bytes<NT>();
     if (lds > raised) {
-        if (hipFuncSetAttribute((const void *)k_mf<GLU, CH, FULL, PT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void *)k_mf<GLU, NT, SM, PT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds) != hipSuccess) return -1;
         raised = lds;
     }
-    SW_LAUNCH((k_mf<GLU, CH, FULL, PT>), dim3(nblocks), dim3(MF_NT), lds, st, A);
+    SW_LAUNCH((k_mf<GLU, NT, SM, PT>), dim3(nblocks), dim3(MF_NTH), lds, st, A);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 template <int GLU, int PT = 0>
 static int mf_dispatch(hipStream_t st, unsigned nblocks, const MfArgs &A) {
-    const int G = A.W.K / SW_RG, Gq = run_lanes(G), CH = Gq < 16 ? Gq : 16;
-    const bool full = G == Gq;
-    if (CH == 16) return full ? mf_go<GLU, 16, 1, PT>(st, nblocks, A) : mf_go<GLU, 16, 0, PT>(st, nblocks, A);
-    if (CH == 8) return full ? mf_go<GLU, 8, 1, PT>(st, nblocks, A) : mf_go<GLU, 8, 0, PT>(st, nblocks, A);
-    if (CH == 4) return full ? mf_go<GLU, 4, 1, PT>(st, nblocks, A) : mf_go<GLU, 4, 0, PT>(st, nblocks, A);
+    const int tt = A.grp.tt ? A.grp.tt : SW_MF_TT;
+#define SW_MF_SM(N_) \
+    (A.W.gs <= 0 ? mf_go<GLU, N_, 0, PT>(st, nblocks, A) \
+     : A.W.gs == SW_RG ? mf_go<GLU, N_, 1, PT>(st, nblocks, A) \
+     : A.W.gs == 2 * SW_RG ? mf_go<GLU, N_, 2, PT>(st, nblocks, A) : mf_go<GLU, N_, 3, PT>(st, nblocks, A))
+    if (tt == 16) return SW_MF_SM(1);
+    if (tt == 32) return SW_MF_SM(2);
+    if (tt == 64) return SW_MF_SM(4);
+#undef SW_MF_SM
     return -1;
 }
-// row blocks per block: the down's 8-chunk row blocks four at a time (as nrb allows;
-// C4 down 1064 -> 968 us); the gate_up's 32-chunk ones one at a time (two measured
-// 1897 -> 1954 us: half the blocks balance worse over the CUs, and a start costs little
-// against 32 chunks)
-#ifndef MF_RBPER_ROWS
+// row blocks per block: the down's short row blocks (K = I) up to four at a time, one start
+// and one drain for all, while that leaves at least 1024 blocks (four per CU) by the launch's
+// bound on its tiles; the gate_up's long ones one at a time
 #define MF_RBPER_ROWS 4
-#endif
-static int mf_rbper(int nrb, int glu) {
-    if (glu) return 1;
+static int mf_rbper(int nrb, int tiles) {
     for (int r = MF_RBPER_ROWS; r > 1; r >>= 1)
-        if (nrb % r == 0) return r;
+        if (nrb % r == 0 && (int64_t)tiles * (nrb / r) >= 1024) return r;
     return 1;
 }
 // shapes: K a multiple of 128 (whole chunks of 4 input groups), tiles listed (items, P),
 // the digits addressed by 32-bit offsets
 static int mf_check(const SwQ4 &W, const SwGroups &g, int &gsh, int dg_rows) {
-    if (W.K % (SW_RG * MF_CG) || !g.items || !g.P || g.ngroups_max <= 0 || !sw_q4_extent_ok(W)) return -1;
+    if (W.K % (SW_RG * 4) || !g.items || !g.P || g.ngroups_max <= 0 || !sw_q4_extent_ok(W)) return -1;
     if (dg_rows <= 0 || (uint64_t)dg_rows * (uint64_t)W.K * 4 > 0xFFFFFFFFull) return -1;
     return sw_q4_gsh(W, gsh);
 }
@@ -535,18 +536,18 @@ static int mf_check(const SwQ4 &W, const SwGroups &g, int &gsh, int dg_rows) {
 int sw_launch_mf_glu(hipStream_t st, SwQ4 W, const uint32_t *dg, const float *xs, int dg_rows, SwGroups g, int I,
                      uint32_t *hdg, float *hxs) {
     int gsh;
-    if (mf_check(W, g, gsh, dg_rows) || I % 64 || W.O != 2 * I) return -1;
-    const int nrb = I / 64;
-    const int rp = mf_rbper(nrb, 1);
+    if (mf_check(W, g, gsh, dg_rows) || I % 128 || W.O != 2 * I) return -1;
+    const int nrb = I / 128;
+    const int rp = 1;
     const MfArgs A = {W, gsh, dg, xs, dg_rows, g, I, nrb, rp, hdg, hxs, nullptr};
     return mf_dispatch<1>(st, (unsigned)(g.ngroups_max * (nrb / rp)), A);
 }
 
 int sw_launch_mf_rows(hipStream_t st, SwQ4 W, const uint32_t *dg, const float *xs, int dg_rows, SwGroups g, float *Y) {
     int gsh;
-    if (mf_check(W, g, gsh, dg_rows) || W.O % 4) return -1;
+    if (mf_check(W, g, gsh, dg_rows) || W.O % 32) return -1;
     const int nrb = (W.O + MF_ROWS - 1) / MF_ROWS;
-    const int rp = mf_rbper(nrb, 0);
+    const int rp = mf_rbper(nrb, g.ngroups_max);
     const MfArgs A = {W, gsh, dg, xs, dg_rows, g, 0, nrb, rp, nullptr, nullptr, Y};
     return mf_dispatch<0>(st, (unsigned)(g.ngroups_max * (nrb / rp)), A);
 }
@@ -557,9 +558,9 @@ int sw_launch_mf_glu_tab(hipStream_t st, SwQ4 W, const SwTab *tab, const uint32_
                          SwGroups g, int I, uint32_t *hdg, float *hxs) {
     int gsh;
     W.E = 1;
-    if (!tab || !hdg || !hxs || mf_check(W, g, gsh, dg_rows) || I % 64 || W.O != 2 * I) return -1;
-    const int nrb = I / 64;
-    const int rp = mf_rbper(nrb, 1);
+    if (!tab || !hdg || !hxs || mf_check(W, g, gsh, dg_rows) || I % 128 || W.O != 2 * I) return -1;
+    const int nrb = I / 128;
+    const int rp = 1;
     const MfArgs A = {W, gsh, dg, xs, dg_rows, g, I, nrb, rp, hdg, hxs, nullptr, tab};
     return mf_dispatch<1, 1>(st, (unsigned)(g.ngroups_max * (nrb / rp)), A);
 }
@@ -567,9 +568,9 @@ int sw_launch_mf_rows_tab(hipStream_t st, SwQ4 W, const SwTab *tab, const uint32
                           SwGroups g, float *Y) {
     int gsh;
     W.E = 1;
-    if (!tab || !Y || mf_check(W, g, gsh, dg_rows) || W.O % 4) return -1;
+    if (!tab || !Y || mf_check(W, g, gsh, dg_rows) || W.O % 32) return -1;
     const int nrb = (W.O + MF_ROWS - 1) / MF_ROWS;
-    const int rp = mf_rbper(nrb, 0);
+    const int rp = mf_rbper(nrb, g.ngroups_max);
     const MfArgs A = {W, gsh, dg, xs, dg_rows, g, 0, nrb, rp, nullptr, nullptr, Y, tab};
     return mf_dispatch<0, 1>(st, (unsigned)(g.ngroups_max * (nrb / rp)), A);
 }

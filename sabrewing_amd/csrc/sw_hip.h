@@ -169,16 +169,28 @@ struct SwGateOpt { int ld, ns; float rs; int wld; float *wsh; int wshld; };
 // the upper bound of the passes of T packed rows in at most min(T, E) groups, tt tokens each
 __host__ __device__ inline int sw_npass_max(int T, int E, int tt) { return (T + (T < E ? T : E) * (tt - 1)) / tt; }
 #define SW_MF_TT 64               // the prefill MFMA kernels' largest token tile
-// the MFMA tiles of a group of n tokens: ceil(n / 64) of them (as 64-token tiles), each
-// of the same whole number of 16-token columns (80 tokens: 48 + 32, not 64 + 16 -- a
-// tail column costs most of what a full tile's staging does)
-__host__ __device__ inline int sw_mf_tile(int n) {
-    const int nt = (n + SW_MF_TT - 1) / SW_MF_TT, ts = ((n + nt - 1) / nt + 15) / 16 * 16;
-    return ts < SW_MF_TT ? ts : SW_MF_TT;
+// The MFMA against dot8 for T packed rows in G groups: from 4.75 rows a group.  dot8's time
+// grows with the rows (24 dots per weight group and row), the MFMA's hardly does up to 16.
+// Measured per layer step, dot8 against the MFMA: C2 at 4.4 rows a group 693 / 720 us, at 5
+// 771 / 730, at 7 1,117 / 837; C1 at 4 114 / 126, at 6 142 / 120; D = 2048, I = 512, E = 256
+// at 4 209 / 193; C5 at 4 900 / 892.
+__host__ __device__ inline bool sw_mf_wins(int64_t T, int64_t G) { return 4 * T >= 19 * G; }
+// tokens per tile of the MFMA launches: 16 (four waves per SIMD) up to 9 rows a group, 32 up
+// to 22, else 64 (each weight expanded once for four columns of tokens).  Measured per layer
+// step with 16 / 32 / 64: C2 at 5 rows a group 730 / 752 / 837 us, at 10 899 / 890 / 1,016, at
+// 27 1,485 / 1,249 / 1,256, at 40 1,903 / 1,700 / 1,473; C1 at 20 182 / 147 / 160, at 31
+// 225 / 206 / 180; C5 at 22 1,636 / 1,374 / 1,393
+__host__ __device__ inline int sw_mf_cols(int64_t T, int64_t G) { return T <= 9 * G ? 16 : T <= 22 * G ? 32 : SW_MF_TT; }
+// the MFMA tiles of a group of n tokens, at most tt each: ceil(n / tt) of them, each of the
+// same whole number of 16-token columns (80 tokens in 64s: 48 + 32, not 64 + 16 -- a tail
+// column costs most of what a full tile's staging does)
+__host__ __device__ inline int sw_mf_tile(int n, int tt) {
+    const int nt = (n + tt - 1) / tt, ts = ((n + nt - 1) / nt + 15) / 16 * 16;
+    return ts < tt ? ts : tt;
 }
 // the token step between the passes (items) of a group of n tokens listed with tt
-// tokens each: tt, or the balanced MFMA tile for tt = SW_MF_TT (the same count of passes)
-__host__ __device__ inline int sw_item_step(int n, int tt) { return tt == SW_MF_TT ? sw_mf_tile(n) : tt; }
+// tokens each: tt, or the balanced MFMA tile from tt = 16 on (the same count of passes)
+__host__ __device__ inline int sw_item_step(int n, int tt) { return tt >= 16 ? sw_mf_tile(n, tt) : tt; }
 // XCD-aware block order: launches deal consecutive block ids to the 8 XCDs in
 // turn; work index w gives XCD k the contiguous range [k n/8, (k+1) n/8) of
 // the first n = 8 floor(nb/8) blocks, so neighbouring work (the passes of one

@@ -1,0 +1,56 @@
+"""The MFMA GEMMs (k_mfma.hip) at the edges of their tiles, through lag_hip_moe_group: groups
+of every size around a column (16 tokens) and a tile (16, 32 or 64 by the average group),
+inputs of 1, 2, 3 and 4 quads of groups and beyond a run, outputs that end in half a row
+block, every scale layout.  dot8 forms the same sums in the same order, so the bits must be
+equal; dot8 itself is checked against the oracle in test_gpu_moe.py."""
+import numpy as np
+import pytest
+
+from sabrewing_amd.backend import Backend
+
+pytestmark = pytest.mark.gpu
+DOT8, MFMA = 1, 2
+
+
+class _Layer:
+    pass
+
+
+def _run(be, L, x, sizes, K, gs):
+    """group g: expert g, sizes[g] rows; every row is its own token (K = 1)"""
+    T = sum(sizes)
+    gexp, gcnt = np.arange(len(sizes), dtype=np.int32), np.array(sizes, np.int32)
+    gbeg = np.concatenate([[0], np.cumsum(gcnt)[:-1]]).astype(np.int32)
+    perm = np.random.default_rng(7).permutation(T).astype(np.int32)      # packed row -> token
+    rowof = np.empty(T, np.int32)
+    rowof[perm] = np.arange(T, dtype=np.int32)
+    w = np.ones((T, 1), np.float32)
+    return be.moe_group(x, L, gexp, gbeg, gcnt, perm, rowof, w, K, gs)
+
+
+@pytest.mark.parametrize("gs", [0, 32, 64, 128])
+@pytest.mark.parametrize("D,I", [(128, 128), (256, 384), (384, 256), (640, 128), (1152, 512)])
+@pytest.mark.parametrize("sizes", [[1, 16, 2, 15, 3], [17, 16, 31, 1, 32], [33, 64, 63, 16, 5], [65, 129, 48, 1, 80]],
+                         ids=["cols16", "cols32", "cols64", "split"])
+def test_mfma_tiles_equal_dot8(be: Backend, gs, D, I, sizes):
+    rng = np.random.default_rng(D + I + gs)
+    E, n = len(sizes), lambda K: K // gs if gs else 1
+    L = _Layer()
+    L.D, L.I = D, I
+    q = lambda r, K: be.upload(rng.integers(0, 256, (r, K // 2), dtype=np.uint8))
+    s = lambda r, K: be.upload(rng.uniform(1e-3, 4e-3, (r, n(K))).astype(np.float32))
+    L.gu_q, L.gu_s, L.dn_q, L.dn_s = q(E * 2 * I, D), s(E * 2 * I, D), q(E * D, I), s(E * D, I)
+    x = rng.standard_normal((sum(sizes), D)).astype(np.float32) * rng.choice([1e-3, 1.0, 30.0], (sum(sizes), 1)).astype(np.float32)
+    x[:, :32] = 0.0                                   # a zero group, and a token of zeros
+    x[1] = 0.0
+    out = {}
+    for mode in (DOT8, MFMA):
+        prev = be.set_grouped_kernel(mode)
+        try:
+            out[mode] = _run(be, L, x, sizes, 1, gs)
+        finally:
+            be.set_grouped_kernel(prev)
+    for b in (L.gu_q, L.gu_s, L.dn_q, L.dn_s):
+        b.free()
+    assert np.isfinite(out[DOT8]).all()
+    assert np.array_equal(out[MFMA].view(np.uint32), out[DOT8].view(np.uint32))
