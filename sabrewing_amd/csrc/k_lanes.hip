@@ -28,9 +28,10 @@
 // Each (row, token) is one lane chain, so a result never depends on the
 // shape of the launch that computed it.
 //
-// Block: 256 threads = 16 rows x 16 lanes; tiles of CC columns of the 16
-// rows (coalesced 16-byte loads) and of up to TS tokens go through LDS, and
-// each token's chains stay in registers across tiles.
+// k_lanes_w streams rows of whole 16-byte pieces (below).  k_lanes16 takes the rest -- the
+// group-scaled int4, odd row lengths, odd addresses: 256 threads = 16 rows x 16 lanes; tiles
+// of CC columns of the 16 rows (coalesced 16-byte loads) and of up to TS tokens go through
+// LDS, and each token's chains stay in registers across tiles.
 #include "sw_hip.h"
 #include "sw_libm.h"
 
@@ -42,8 +43,8 @@ enum { WK_BF16 = 0, WK_I8 = 1, WK_I4 = 2, WK_I4G = 3 };
 __device__ __forceinline__ float bf16_widen(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
 // a denormal to a signed zero (the DAZ / FTZ of vdpbf16ps)
 __device__ __forceinline__ float flush_dn(float v) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, v);
-    return (u & 0x7F800000u) ? v : __builtin_bit_cast(float, u & 0x80000000u);
+    // (one class test: 0x90 are the two subnormal classes)
+    return __builtin_amdgcn_classf(v, 0x90) ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0x80000000u) : v;
 }
 // vcvtne2ps2bf16 of one float, widened back to f32
 __device__ __forceinline__ float round_bf16_ne(float f) {
@@ -89,6 +90,27 @@ __device__ __forceinline__ float reduce16_lanes(float v) {
     v = v + __shfl_xor(v, 4, 16);
     v = v + __shfl_xor(v, 2, 16);
     return v + __shfl_xor(v, 1, 16);
+}
+
+// row o of token s out: the scalar tail of the columns past imain, then the row scale
+template <int WK, int DP>
+__device__ __forceinline__ void lanes_out(const LanesArgs &A, float sm, int s, int o, int imain) {
+    const float *xs = A.x + (size_t)s * A.ldx;
+    const uint8_t *wr = (const uint8_t *)A.W + (size_t)o * ((size_t)A.I * WElem<WK == WK_I4G ? WK_I4 : WK>::bits / 8);
+    if constexpr (WK == WK_I4) {                       // the byte tail of c/moe_quant.h:105-108
+        for (int i = imain; i + 1 < A.I; i += 2) {
+            const uint8_t b = wr[i >> 1];
+            const float lo = (float)((int)(b & 15) - 8), hi = (float)((int)(b >> 4) - 8);
+            sm = sm + __builtin_fmaf(xs[i], lo, xs[i + 1] * hi);
+        }
+    } else if constexpr (!DP) {
+        for (int i = imain; i < A.I; i++) {
+            const float w = WK == WK_BF16 ? bf16_widen(((const uint16_t *)wr)[i]) : (float)((const int8_t *)wr)[i];
+            sm = __builtin_fmaf(xs[i], w, sm);
+        }
+    }
+    if (WK != WK_I4G && A.scale) sm = sm * A.scale[o];
+    A.y[(size_t)s * A.ldy + o] = sm;
 }
 
 template <int WK, int DP, int TS>
@@ -219,28 +241,182 @@ __global__ __launch_bounds__(256) void k_lanes16(LanesArgs A) {
     for (int t = 0; t < TS; t++) {
         float sm = WK == WK_I4G ? acc[t] : reduce16_lanes(acc[t]);    // I4G: lane 0 holds the row's sum
         if (j == 0 && t < ns && o < O) {
-            const float *xs = A.x + (size_t)(s0 + t) * A.ldx;
-            const uint8_t *wr = W + (size_t)o * rowb;
-            if constexpr (WK == WK_I4) {               // the byte tail of c/moe_quant.h:105-108
-                for (int i = imain; i + 1 < I; i += 2) {
-                    const uint8_t b = wr[i >> 1];
-                    const float lo = (float)((int)(b & 15) - 8), hi = (float)((int)(b >> 4) - 8);
-                    sm = sm + __builtin_fmaf(xs[i], lo, xs[i + 1] * hi);
-                }
-            } else if constexpr (!DP) {
-                for (int i = imain; i < I; i++) {
-                    const float w = WK == WK_BF16 ? bf16_widen(((const uint16_t *)wr)[i]) : (float)((const int8_t *)wr)[i];
-                    sm = __builtin_fmaf(xs[i], w, sm);
-                }
-            }
-            if (WK != WK_I4G && A.scale) sm = sm * A.scale[o];
-            A.y[(size_t)(s0 + t) * A.ldy + o] = sm;
+            lanes_out<WK, DP>(A, sm, s0 + t, o, imain);
         }
     }
 }
 
+// ---- rows in 16-byte pieces, streamed by waves (every contract but I4G) ----
+// A wave owns 4 rows; lane 16 r + j runs chain j of row r for up to TS tokens.  Per step it
+// loads 16 bytes per lane -- 16 EPL consecutive columns of each row, one contiguous KB, PF
+// steps in flight -- and turns them through its own LDS into the chains' order (one b128
+// write, then per element one 2-byte (bf16), 1-byte (int) or, for DP, per pair one 4-byte
+// read).  The tokens' x goes through LDS for the whole block, LW_XC columns at a time in two
+// buffers, stored by chain (xt[t][j][m], so a lane reads four of its chain's values at once);
+// one barrier per LW_XC columns.  What bounds it: HBM latency at one token (1 KB x PF per
+// wave in flight), LDS reads of x at 8 (8 values of 16 bytes per 8 weights and 32 fmas).
+// k_lanes16, which every shape took before, walked 256-column tiles with two barriers each,
+// nothing in flight across them and one LDS read of x per fma: bf16 4096 x 4096, 16 tokens
+// 151 -> 35 us a launch; the gated shared experts at 4 tokens (DP, gate and up of 4096 x 4096
+// each, two downs of 4096 x 2048) 64 -> 30 and 33 -> 14 us a launch.
+#define LW_XC 512
+#define LW_XM (LW_XC / 16)         // chain elements of an x chunk
+#define LW_XS (LW_XM + 4)          // floats per (token, chain) in LDS
+#define LW_WS 288                  // bytes per row of a wave's weight step in LDS
+#define LW_WAVES 4
+template <int WK, int DP, int TS>
+__global__ __launch_bounds__(64 * LW_WAVES) void k_lanes_w(LanesArgs A) {
+    constexpr int EPL = 128 / WElem<WK>::bits;         // elements of a lane's 16 bytes
+    constexpr int CS = 16 * EPL, SPC = LW_XC / CS;     // columns per step, steps per x chunk
+    constexpr int RC = WK == WK_BF16 ? 2 : 4;          // x chunks whose weight steps are in flight
+    constexpr int PF = RC * SPC;
+    constexpr int NTH = 64 * LW_WAVES, XR = (TS * LW_XC / 4 + NTH - 1) / NTH;
+    extern __shared__ __align__(16) uint8_t lw_lds[];
+    float *xt = (float *)lw_lds;                       // [2][TS][16][LW_XS]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane >> 4, j = lane & 15;
+    uint8_t *wl = lw_lds + 2 * TS * 16 * LW_XS * 4 + wave * 2 * 4 * LW_WS;   // [2][4][LW_WS]
+    const int I = A.I, O = A.O, S = A.S;
+    const int o = (blockIdx.x * LW_WAVES + wave) * 4 + r, s0 = blockIdx.y * TS, ns = min(TS, S - s0);
+    const int imain = WK == WK_I4 ? I & ~31 : I & ~15;
+    const int nst = (imain + CS - 1) / CS, nch = (imain + LW_XC - 1) / LW_XC;
+    const size_t rowb = (size_t)I * WElem<WK>::bits / 8;
+    const uint8_t *wr = (const uint8_t *)A.W + (size_t)min(o, O - 1) * rowb;
+    const int lastp = imain * WElem<WK>::bits / 128 - 1;    // the row's last whole 16-byte piece
+    // (unconditional: a piece past the end re-reads the last one, whose elements are not used)
+    auto wld = [&](int st) { return *(const sw_u32x4 *)(wr + 16 * (size_t)max(min(st * 16 + j, lastp), 0)); };
+    sw_f32x4 xr[XR];
+    auto xload = [&](int c) {                          // float4 f of a chunk: token f / 128, columns 4 (f % 128)
+#pragma unroll
+        for (int u = 0; u < XR; u++) {
+            const int f = u * NTH + tid, t = min(f / (LW_XC / 4), TS - 1), k = c * LW_XC + 4 * (f % (LW_XC / 4));
+            xr[u] = *(const sw_f32x4 *)(A.x + (size_t)(s0 + min(t, ns - 1)) * A.ldx + min(k, imain - 4));
+        }
+    };
+    auto xstore = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < XR; u++) {
+            const int f = u * NTH + tid, t = f / (LW_XC / 4), k4 = 4 * (f % (LW_XC / 4));
+            if (TS * LW_XC / 4 % NTH == 0 || t < TS)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int k = k4 + i;
+                    const int ch = DP ? (k & 31) >> 1 : k & 15, m = DP ? 2 * (k >> 5) + (k & 1) : k >> 4;
+                    xt[((buf * TS + t) * 16 + ch) * LW_XS + m] = DP ? round_bf16_ne(xr[u][i]) : xr[u][i];
+                }
+        }
+    };
+    float acc[TS];
+#pragma unroll
+    for (int t = 0; t < TS; t++) acc[t] = 0.f;
+    sw_u32x4 ring[PF];
+#pragma unroll
+    for (int u = 0; u < PF; u++) ring[u] = wld(u);
+    xload(0);
+    xstore(0);
+    __syncthreads();
+    // elements m .. m + 3 of the step (chain elements m0 + m .. of the x chunk in buffer buf)
+    auto four = [&](const uint8_t *row, int m, const float *xc) {
+        float w[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if constexpr (DP) {                        // pair q = (m + i) / 2 of columns 32 q + 2 j: slot 0 even, 1 odd
+                const uint32_t v = *(const uint32_t *)(row + ((m + i) >> 1) * 64 + 4 * j);
+                w[i] = flush_dn((i & 1) ? __builtin_bit_cast(float, v & 0xFFFF0000u) : bf16_widen(v & 0xFFFFu));
+            } else {
+                w[i] = w_at<WK>(row, 16 * (m + i) + j);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TS; t++) {
+            const sw_f32x4 xv = *(const sw_f32x4 *)(xc + t * 16 * LW_XS + m);
+            if constexpr (DP) {                        // the odd column first
+                acc[t] = flush_dn(__builtin_fmaf(xv[1], w[1], acc[t]));
+                acc[t] = flush_dn(__builtin_fmaf(xv[0], w[0], acc[t]));
+                acc[t] = flush_dn(__builtin_fmaf(xv[3], w[3], acc[t]));
+                acc[t] = flush_dn(__builtin_fmaf(xv[2], w[2], acc[t]));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[t] = __builtin_fmaf(xv[i], w[i], acc[t]);
+            }
+        }
+    };
+    for (int c0 = 0; c0 < nch; c0 += RC) {
+#pragma unroll
+        for (int h = 0; h < RC; h++) {
+            const int c = c0 + h;
+            if (c >= nch) break;                       // uniform
+            xload(min(c + 1, nch - 1));
+            const float *xc = xt + (((c & 1) * TS) * 16 + j) * LW_XS;
+#pragma unroll
+            for (int p = 0; p < SPC; p++) {
+                const int st = c * SPC + p, u = h * SPC + p;
+                if (st >= nst) break;                  // uniform
+                uint8_t *row = wl + ((p & 1) * 4 + r) * LW_WS;
+                *(sw_u32x4 *)(row + 16 * j) = ring[u];
+                ring[u] = wld(st + PF);
+                __builtin_amdgcn_sched_barrier(0);
+                lanes_wave_sync();
+                const int mc = min(EPL, (imain - st * CS) / 16);
+                if (mc == EPL) {
+#pragma unroll
+                    for (int m = 0; m < EPL; m += 4) four(row, m, xc + p * EPL);
+                } else {                               // the row's last columns: one (DP: two) at a time
+                    for (int m = 0; m < mc; m += DP ? 2 : 1)
+#pragma unroll
+                        for (int t = 0; t < TS; t++) {
+                            const float *xm = xc + p * EPL + t * 16 * LW_XS + m;
+                            if constexpr (DP) {
+                                const uint32_t v = *(const uint32_t *)(row + (m >> 1) * 64 + 4 * j);
+                                acc[t] = flush_dn(__builtin_fmaf(xm[1], flush_dn(__builtin_bit_cast(float, v & 0xFFFF0000u)), acc[t]));
+                                acc[t] = flush_dn(__builtin_fmaf(xm[0], flush_dn(bf16_widen(v & 0xFFFFu)), acc[t]));
+                            } else {
+                                acc[t] = __builtin_fmaf(xm[0], w_at<WK>(row, 16 * m + j), acc[t]);
+                            }
+                        }
+                }
+                lanes_wave_sync();                     // read before the buffer's next write
+            }
+            xstore((c + 1) & 1);                       // (read by no wave since the last barrier)
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TS; t++) {
+        const float sm = reduce16_lanes(acc[t]);
+        if (j == 0 && t < ns && o < O) lanes_out<WK, DP>(A, sm, s0 + t, o, imain);
+    }
+}
+
+template <int WK, int DP, int TS>
+static void launch_lanes_w(hipStream_t st, const LanesArgs &A) {
+    const size_t lds = (size_t)2 * TS * 16 * LW_XS * 4 + LW_WAVES * 2 * 4 * LW_WS;
+    SW_LAUNCH((k_lanes_w<WK, DP, TS>), dim3((A.O + 4 * LW_WAVES - 1) / (4 * LW_WAVES), (A.S + TS - 1) / TS), dim3(64 * LW_WAVES),
+              lds, st, A);
+}
+// whole 16-byte pieces: rows of W and of x at 16-byte strides and addresses, at least one
+// chain step in a row
+static bool lanes_w_ok(const LanesArgs &A, int bits) {
+    return (size_t)A.I * bits / 8 % 16 == 0 && (size_t)A.I * bits % 8 == 0 && ((uintptr_t)A.W & 15) == 0 &&
+           ((uintptr_t)A.x & 15) == 0 && A.ldx % 4 == 0 && A.I >= 32;
+}
+
 template <int WK, int DP>
 static void launch_lanes(hipStream_t st, const LanesArgs &A) {
+    if constexpr (WK != WK_I4G) {
+        if (lanes_w_ok(A, WElem<WK>::bits)) {
+            // tokens per pass: the most (each weight turned once for all of them) that still give
+            // 512 blocks, two waves per SIMD -- one alone issues at half rate (bf16 4096 x 4096 at 8
+            // tokens, whole call: 66 us with 256 blocks, 58 with 512, 57 with 1024; 24 tokens at
+            // 6144 rows no difference, 4 tokens there 55 / 52 / 56)
+            int ts = A.S >= 8 ? 8 : A.S >= 3 ? 4 : A.S;
+            while (ts > 1 && (int64_t)((A.O + 4 * LW_WAVES - 1) / (4 * LW_WAVES)) * ((A.S + ts - 1) / ts) < 512) ts >>= 1;
+            if (ts == 8) launch_lanes_w<WK, DP, 8>(st, A);
+            else if (ts == 4) launch_lanes_w<WK, DP, 4>(st, A);
+            else if (ts == 2) launch_lanes_w<WK, DP, 2>(st, A);
+            else launch_lanes_w<WK, DP, 1>(st, A);
+            return;
+        }
+    }
     const int ts = A.S >= 16 ? 16 : A.S >= 8 ? 8 : A.S >= 4 ? 4 : 1;
     const dim3 block(256);
     if (ts == 16) SW_LAUNCH((k_lanes16<WK, DP, 16>), dim3((A.O + 15) / 16, (A.S + 15) / 16), block, 0, st, A);

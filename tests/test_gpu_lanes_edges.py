@@ -1,0 +1,80 @@
+"""The host-activation matmuls where their two kernels meet (k_lanes.hip): rows in whole
+16-byte pieces are streamed by waves, everything else takes the general tiles.  Inputs around
+a step (128, 256 or 512 columns by the weight type), an x chunk (512 columns) and the scalar
+tail, outputs around a wave's 4 rows and a block's 16, tokens around the passes of 1, 2, 4 and
+8; a weight address off by one element takes the general kernel.  All bit for bit the
+oracle's, whose matmuls are pinned to the compiled reference."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+SHAPES = [(32, 1), (64, 5), (96, 16), (160, 17), (512, 3), (528, 20), (544, 33), (1024, 18), (1056, 7), (1504, 67)]
+TOKENS = [1, 2, 3, 4, 7, 8, 9, 17]
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+class _At:
+    def __init__(self, buf, off):
+        self.p = int(buf) + off
+
+    def __int__(self):
+        return self.p
+
+
+def _x(rng, S, I):
+    x = rng.standard_normal((S, I)).astype(np.float32)
+    x[0, ::7] = 0.0
+    x[-1, 1::5] *= np.float32(1e-30)                  # products below the normal range
+    return x
+
+
+@pytest.mark.parametrize("I,O", SHAPES + [(40, 9), (536, 19)])
+def test_bf16(be, orc, I, O):
+    rng = np.random.default_rng(I * 131 + O)
+    Wb = orc.to_bf16(rng.standard_normal((O, I)).astype(np.float32) * np.float32(0.02)).reshape(O, I)
+    Wb[0, :3] = [1, 0x8001, 0x7F]                     # denormal weights
+    pad = np.zeros(O * I + 1, np.uint16)
+    pad[1:] = Wb.reshape(-1)
+    d0, d1 = be.upload(Wb), be.upload(pad)
+    for S in TOKENS:
+        x = _x(rng, S, I)
+        for got in (be.matmul_bf16(x, d0, O), be.matmul_bf16(x, _At(d1, 2), O)):
+            assert np.array_equal(bits(got), bits(orc.matmul_bf16(x, Wb))), (S, I, O)
+        for got in (be.matmul_bf16_rx(x, d0, O), be.matmul_bf16_rx(x, _At(d1, 2), O)):
+            assert np.array_equal(bits(got), bits(orc.matmul_bf16_rx(x, Wb))), (S, I, O)
+    d0.free(); d1.free()
+
+
+@pytest.mark.parametrize("I,O", SHAPES + [(1040, 6)])
+def test_q8(be, orc, I, O):
+    rng = np.random.default_rng(I * 137 + O)
+    q = rng.integers(-127, 128, (O, I)).astype(np.int8)
+    sc = rng.uniform(1e-3, 2e-3, O).astype(np.float32)
+    pad = np.zeros(O * I + 1, np.int8)
+    pad[1:] = q.reshape(-1)
+    d0, d1, ds = be.upload(q), be.upload(pad), be.upload(sc)
+    for S in TOKENS:
+        x = _x(rng, S, I)
+        for got in (be.matmul_q8(x, d0, ds, O), be.matmul_q8(x, _At(d1, 1), ds, O)):
+            assert np.array_equal(bits(got), bits(orc.matmul_q8(x, q, sc, 0))), (S, I, O)
+    for b in (d0, d1, ds):
+        b.free()
+
+
+@pytest.mark.parametrize("I,O", SHAPES)
+def test_q4(be, orc, I, O):
+    rng = np.random.default_rng(I * 139 + O)
+    p = rng.integers(0, 256, (O, I // 2), dtype=np.uint8)
+    sc = rng.uniform(1e-3, 2e-3, O).astype(np.float32)
+    pad = np.zeros(O * I // 2 + 1, np.uint8)
+    pad[1:] = p.reshape(-1)
+    d0, d1, ds = be.upload(p), be.upload(pad), be.upload(sc)
+    for S in TOKENS:
+        x = _x(rng, S, I)
+        for got in (be.matmul_q4(x, d0, ds, O, 0), be.matmul_q4(x, _At(d1, 1), ds, O, 0)):
+            assert np.array_equal(bits(got), bits(orc.matmul_q4(x, p, sc))), (S, I, O)
+    for b in (d0, d1, ds):
+        b.free()
