@@ -20,7 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 HIP_SOURCES = ["backend_hip.hip", "k_dot8.hip", "k_mfma.hip", "k_idot.hip", "k_shared.hip", "k_route.hip", "coli_hip.hip",
-               "k_gen.hip", "k_glue.hip", "k_lanes.hip"]
+               "k_gen.hip", "k_glue.hip", "k_lanes.hip", "k_xfer.hip"]
 HIP_LIB = os.path.join(HERE, "libsabrewing_hip.so")
 LOADER_LIB = os.path.join(HERE, "libsabrewing_loader.so")
 ARCH = "gfx950"

@@ -274,12 +274,12 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
     if (mf) { o_xd = cv.take((size_t)S * (D / 32) * 128); o_hd = cv.take((size_t)T * (I / 32) * 128); }
     if (grow_dev(g_arena, cv.off)) return -1;
     char *A = (char *)g_arena.p;
-    // one pinned blob: x | gexp gbeg gcnt grow rowof w [| items P]
-    const size_t xn = (size_t)S * D * 4;
-    if (grow_pinned(g_hin, xn + idxn) || grow_pinned(g_hout, (size_t)S * D * 4)) return -1;
+    // one pinned image of the arena's head, one upload: x | gexp gbeg gcnt grow rowof w [| items P]
+    const size_t xn = (size_t)S * D * 4, up = o_idx + idxn;
+    if (grow_pinned(g_hin, up) || grow_pinned(g_hout, (size_t)S * D * 4)) return -1;
     char *H = (char *)g_hin.p;
     memcpy(H, x, xn);
-    int *hi = (int *)(H + xn);
+    int *hi = (int *)(H + o_idx);
     memcpy(hi, gexp, (size_t)G * 4);
     memcpy(hi + G, gbeg, (size_t)G * 4);
     memcpy(hi + 2 * G, gcnt, (size_t)G * 4);
@@ -292,8 +292,7 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
             for (int t0 = 0; t0 < gcnt[i]; t0 += sw_mf_tile(gcnt[i], tt)) it[n++] = (t0 << 10) | i;
         it[n] = n;
     }
-    CK(hipMemcpyAsync(A + o_x, H, xn, hipMemcpyHostToDevice, g_st), "x upload");
-    CK(hipMemcpyAsync(A + o_idx, H + xn, idxn, hipMemcpyHostToDevice, g_st), "index upload");
+    CK(sw_xfer(g_st, A, H, up, hipMemcpyHostToDevice), "input upload");
     const int *d_gexp = (const int *)(A + o_idx), *d_gbeg = d_gexp + G, *d_gcnt = d_gexp + 2 * G;
     const int *d_grow = d_gexp + 3 * G, *d_rowof = d_grow + T;
     const float *d_w = (const float *)(d_rowof + T);
@@ -326,7 +325,7 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
                               (float *)(A + o_out), 0)) return fail_msg("combine launch");
         res = (const float *)(A + o_out);
     }
-    CK(hipMemcpyAsync(g_hout.p, res, (size_t)S * D * 4, hipMemcpyDeviceToHost, g_st), "result download");
+    CK(sw_xfer(g_st, g_hout.p, res, (size_t)S * D * 4, hipMemcpyDeviceToHost), "result download");
     CK(hipStreamSynchronize(g_st), "stream sync");
     memcpy(outh, g_hout.p, (size_t)S * D * 4);
     if (g_prof) prof_flush();
@@ -387,11 +386,11 @@ static int lanes_host(float *y, const float *x, const void *W, int wkind, int dp
     if (grow_dev(g_arena, cv.off) || grow_pinned(g_hin, (size_t)S * I * 4) || grow_pinned(g_hout, (size_t)S * O * 4)) return -1;
     char *A = (char *)g_arena.p;
     memcpy(g_hin.p, x, (size_t)S * I * 4);
-    CK(hipMemcpyAsync(A + o_x, g_hin.p, (size_t)S * I * 4, hipMemcpyHostToDevice, g_st), "x upload");
+    CK(sw_xfer(g_st, A + o_x, g_hin.p, (size_t)S * I * 4, hipMemcpyHostToDevice), "x upload");
     { PROF("lanes16");
       if (sw_launch_lanes16(g_st, W, wkind, dp, (const float *)scale, (const float *)(A + o_x), S, I, O, (float *)(A + o_y), gs))
           return fail_msg("lanes launch (shape unsupported?)"); }
-    CK(hipMemcpyAsync(g_hout.p, A + o_y, (size_t)S * O * 4, hipMemcpyDeviceToHost, g_st), "result download");
+    CK(sw_xfer(g_st, g_hout.p, A + o_y, (size_t)S * O * 4, hipMemcpyDeviceToHost), "result download");
     CK(hipStreamSynchronize(g_st), "stream sync");
     memcpy(y, g_hout.p, (size_t)S * O * 4);
     if (g_prof) prof_flush();
@@ -959,10 +958,10 @@ extern "C" int lag_hip_moe_block(const LagHipMoeDesc *d, const LagHipMoeWeights 
     if (grow_dev(dx, n) || grow_dev(dout, n) || grow_pinned(g_hin, n) || grow_pinned(g_hout, n)) return -1;
     memcpy(g_hin.p, x, n);
     memcpy(g_hout.p, out, n);
-    CK(hipMemcpyAsync(dx.p, g_hin.p, n, hipMemcpyHostToDevice, g_st), "x upload");
-    CK(hipMemcpyAsync(dout.p, g_hout.p, n, hipMemcpyHostToDevice, g_st), "out upload");
+    CK(sw_xfer(g_st, dx.p, g_hin.p, n, hipMemcpyHostToDevice), "x upload");
+    CK(sw_xfer(g_st, dout.p, g_hout.p, n, hipMemcpyHostToDevice), "out upload");
     if (lag_hip_moe_forward(d, w, (const float *)dx.p, (float *)dout.p, S)) return -1;
-    CK(hipMemcpyAsync(g_hout.p, dout.p, n, hipMemcpyDeviceToHost, g_st), "out download");
+    CK(sw_xfer(g_st, g_hout.p, dout.p, n, hipMemcpyDeviceToHost), "out download");
     CK(hipStreamSynchronize(g_st), "stream sync");
     memcpy(out, g_hout.p, n);
     if (g_prof) prof_flush();

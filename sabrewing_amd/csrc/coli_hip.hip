@@ -153,7 +153,7 @@ int collect(ColiHipTensor *const *gates, ColiHipTensor *const *ups, ColiHipTenso
 
 // device scratch of a group call over T rows: x | gexp gbeg gcnt grow/items | tab |
 // limbs (dot8) or digits (MFMA) of x and of h, with their factors | y
-struct GLay { size_t x, ints, tab, xl, xs, hl, hs, y, end; };
+struct GLay { size_t x, ints, tab, in_end, xl, xs, hl, hs, y, end; };
 // (T rows through the projections, xrows rows of x, ints: 3 per group + nextra)
 GLay glay(const Groups &G, int T, int xrows, int nextra = 0, bool mf = false) {
     Carve cv;
@@ -162,6 +162,7 @@ GLay glay(const Groups &G, int T, int xrows, int nextra = 0, bool mf = false) {
     L.x = cv.take((size_t)xrows * G.D * 4);
     L.ints = cv.take((size_t)(3 * G.count + nextra) * 4);
     L.tab = cv.take((size_t)G.count * sizeof(SwTab));
+    L.in_end = cv.off;                                     // x, ints and tab: one upload from an image of this head
     L.xl = cv.take((size_t)xrows * (G.D / 32) * per_group);
     L.xs = cv.take((size_t)xrows * (G.D / 32) * 4);
     L.hl = cv.take((size_t)T * (G.I / 32) * per_group);
@@ -173,14 +174,13 @@ GLay glay(const Groups &G, int T, int xrows, int nextra = 0, bool mf = false) {
 // the f16 MFMA GEMMs from 8 rows a group on (the lag family's groups are many, and take them
 // from fewer): whole quads of 4 input groups
 bool use_mf(const Groups &G) { return G.D % 128 == 0 && G.I % 128 == 0 && G.total >= 8 * G.count; }
-size_t meta_bytes(const Groups &G, int T) { return (size_t)(3 * G.count + T) * 4 + (size_t)G.count * sizeof(SwTab); }
-// the host image of the ints and the table: gexp = 0..count-1 (the table index),
-// gbeg, gcnt, grow (or nothing), then the table
-void pack_meta(const Groups &G, const int *grow, int T, char *dst) {
-    int *h = (int *)dst;
+// the ints and the table in the host image H of the scratch's head: gexp = 0..count-1 (the
+// table index), gbeg, gcnt, n further ints (grow, or the MFMA tiles); the table
+void pack_meta(const Groups &G, const GLay &L, const int *more, int n, char *H) {
+    int *h = (int *)(H + L.ints);
     for (int c = 0; c < G.count; c++) { h[c] = c; h[G.count + c] = G.beg[c]; h[2 * G.count + c] = G.cnt[c]; }
-    if (grow) memcpy(h + 3 * G.count, grow, (size_t)T * 4);
-    memcpy(dst + (size_t)(3 * G.count + T) * 4, G.tab.data(), (size_t)G.count * sizeof(SwTab));
+    if (n) memcpy(h + 3 * G.count, more, (size_t)n * 4);
+    memcpy(H + L.tab, G.tab.data(), (size_t)G.count * sizeof(SwTab));
 }
 
 // the four launches: limbs of xrows rows, gate/up + GLU, down -> y [T][D]
@@ -242,8 +242,8 @@ int group_sync(const Groups &G, float *y, const float *x) {
     }
     const int ni = (int)items.size();
     const GLay L = glay(G, T, T, ni, mf);
-    const size_t xb = (size_t)T * G.D * 4, ib = (size_t)(3 * G.count + ni) * 4, mb = ib + (size_t)G.count * sizeof(SwTab);
-    if (!grow(c, c->arena, L.end) || !grow_pinned(c, c->hin, c->hin_cap, xb + mb) ||
+    const size_t xb = (size_t)T * G.D * 4;
+    if (!grow(c, c->arena, L.end) || !grow_pinned(c, c->hin, c->hin_cap, L.in_end) ||
         !grow_pinned(c, c->hout, c->hout_cap, xb))
         return 0;
     char *A = (char *)c->arena.p, *H = (char *)c->hin;
@@ -252,23 +252,14 @@ int group_sync(const Groups &G, float *y, const float *x) {
     if (prof && !c->prof[0])
         for (auto &e : c->prof)
             if (!ok(hipEventCreate(&e), "profile event")) return 0;
-    memcpy(H, x, xb);
-    pack_meta(G, nullptr, 0, H + xb);                      // gexp gbeg gcnt, then the table
-    if (mf) {                                              // the tiles between the ints and the table
-        memmove(H + xb + ib, H + xb + (size_t)(3 * G.count) * 4, (size_t)G.count * sizeof(SwTab));
-        memcpy(H + xb + (size_t)(3 * G.count) * 4, items.data(), (size_t)ni * 4);
-    }
+    memcpy(H + L.x, x, xb);
+    pack_meta(G, L, items.data(), ni, H);                  // (the MFMA tiles after gexp gbeg gcnt)
     if (prof) (void)hipEventRecord(c->prof[0], c->st);
-    // the table follows the ints in the image; in the arena it has its own aligned slot
-    if (!ok(hipMemcpyAsync(A + L.x, H, xb, hipMemcpyHostToDevice, c->st), "expert group input upload") ||
-        !ok(hipMemcpyAsync(A + L.ints, H + xb, ib, hipMemcpyHostToDevice, c->st), "expert group descriptors") ||
-        !ok(hipMemcpyAsync(A + L.tab, H + xb + ib, (size_t)G.count * sizeof(SwTab), hipMemcpyHostToDevice, c->st),
-            "expert group table"))
-        return 0;
+    if (!ok(sw_xfer(c->st, A, H, L.in_end, hipMemcpyHostToDevice), "expert group input upload")) return 0;
     if (prof) (void)hipEventRecord(c->prof[1], c->st);
     if (mf ? !launch_group_mf(c, G, A, L, ni - 1, tt) : !launch_group(c, G, A, L, T, T, false)) return 0;
     if (prof) (void)hipEventRecord(c->prof[2], c->st);
-    if (!ok(hipMemcpyAsync(c->hout, A + L.y, xb, hipMemcpyDeviceToHost, c->st), "expert group output download")) return 0;
+    if (!ok(sw_xfer(c->st, c->hout, A + L.y, xb, hipMemcpyDeviceToHost), "expert group output download")) return 0;
     if (prof) (void)hipEventRecord(c->prof[3], c->st);
     if (!ok(hipStreamSynchronize(c->st), "expert group synchronize")) return 0;
     memcpy(y, c->hout, xb);
@@ -587,9 +578,9 @@ extern "C" int coli_hip_matmul(ColiHipTensor **tensor, float *y, const float *x,
         return 0;
     char *A = (char *)c->arena.p;
     memcpy(c->hin, x, xb);
-    if (!ok(hipMemcpyAsync(A + ox, c->hin, xb, hipMemcpyHostToDevice, c->st), "input upload") ||
+    if (!ok(sw_xfer(c->st, A + ox, c->hin, xb, hipMemcpyHostToDevice), "input upload") ||
         !gemm_dev(c, t, (float *)(A + oy), (const float *)(A + ox), S) ||
-        !ok(hipMemcpyAsync(c->hout, A + oy, yb, hipMemcpyDeviceToHost, c->st), "output download") ||
+        !ok(sw_xfer(c->st, c->hout, A + oy, yb, hipMemcpyDeviceToHost), "output download") ||
         !ok(hipStreamSynchronize(c->st), "matmul synchronize"))
         return 0;
     memcpy(y, c->hout, yb);
@@ -634,19 +625,16 @@ extern "C" int coli_hip_expert_group_issue(ColiHipTensor *const *gates, ColiHipT
     if (c->pending || !select_ctx(c)) return 0;
     const int T = G.total;
     const GLay L = glay(G, T, T);
-    const size_t xb = (size_t)T * G.D * 4, mb = meta_bytes(G, 0);
-    if (!grow(c, c->arena, L.end) || !grow_pinned(c, c->hiss_in, c->hiss_in_cap, xb + mb) ||
+    const size_t xb = (size_t)T * G.D * 4;
+    if (!grow(c, c->arena, L.end) || !grow_pinned(c, c->hiss_in, c->hiss_in_cap, L.in_end) ||
         !grow_pinned(c, c->hiss_out, c->hiss_out_cap, xb))
         return 0;
     char *A = (char *)c->arena.p, *H = (char *)c->hiss_in;
-    memcpy(H, x, xb);
-    pack_meta(G, nullptr, 0, H + xb);
-    if (!ok(hipMemcpyAsync(A + L.x, H, xb, hipMemcpyHostToDevice, c->st), "expert group issue upload") ||
-        !ok(hipMemcpyAsync(A + L.ints, H + xb, (size_t)(3 * G.count) * 4, hipMemcpyHostToDevice, c->st), "issue descriptors") ||
-        !ok(hipMemcpyAsync(A + L.tab, H + xb + (size_t)(3 * G.count) * 4, (size_t)G.count * sizeof(SwTab),
-                           hipMemcpyHostToDevice, c->st), "issue table") ||
+    memcpy(H + L.x, x, xb);
+    pack_meta(G, L, nullptr, 0, H);
+    if (!ok(sw_xfer(c->st, A, H, L.in_end, hipMemcpyHostToDevice), "expert group issue upload") ||
         !launch_group(c, G, A, L, T, T, false) ||
-        !ok(hipMemcpyAsync(c->hiss_out, A + L.y, xb, hipMemcpyDeviceToHost, c->st), "expert group issue download"))
+        !ok(sw_xfer(c->st, c->hiss_out, A + L.y, xb, hipMemcpyDeviceToHost), "expert group issue download"))
         return 0;
     c->pending = 1;
     count_group(G);
@@ -692,17 +680,15 @@ extern "C" int coli_hip_expert_group_resident_issue(ColiHipTensor *const *gates,
     if (!grow(c, c->res, Lc.end + (size_t)G.D * 4 + 256)) return 0;
     // the pinned meta image: wait until the previous issue's copy of it has run
     if (c->ev_res_live && !ok(hipEventSynchronize(c->ev_res), "resident meta wait")) return 0;
-    if (!grow_pinned(c, c->hres, c->hres_cap, meta_bytes(cap, 64))) return 0;
+    if (!grow_pinned(c, c->hres, c->hres_cap, Lc.in_end)) return 0;
     char *A = (char *)c->res.p, *H = (char *)c->hres;
-    pack_meta(G, zeros.data(), T, H);
+    pack_meta(G, L, zeros.data(), T, H);                   // (x comes from the device)
     float *partial = (float *)(A + ((Lc.end + 255) & ~(size_t)255));
     const bool same = home_device == G.device;
     hipError_t xe = same ? hipMemcpyAsync(A + L.x, x_src_dev, (size_t)G.D * 4, hipMemcpyDeviceToDevice, c->st)
                          : hipMemcpyPeerAsync(A + L.x, G.device, x_src_dev, home_device, (size_t)G.D * 4, c->st);
     if (!ok(xe, "resident group x copy") ||
-        !ok(hipMemcpyAsync(A + L.ints, H, (size_t)(3 * G.count + T) * 4, hipMemcpyHostToDevice, c->st), "resident descriptors") ||
-        !ok(hipMemcpyAsync(A + L.tab, H + (size_t)(3 * G.count + T) * 4, (size_t)G.count * sizeof(SwTab),
-                           hipMemcpyHostToDevice, c->st), "resident table") ||
+        !ok(sw_xfer(c->st, A + L.ints, H + L.ints, L.in_end - L.ints, hipMemcpyHostToDevice), "resident descriptors") ||
         !ok(hipEventRecord(c->ev_res, c->st), "resident meta event"))
         return 0;
     c->ev_res_live = 1;

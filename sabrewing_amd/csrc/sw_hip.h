@@ -394,6 +394,8 @@ int sw_launch_argmax(hipStream_t st, const float *logits, int S, int V, int *tok
 // the shared expert of a batch on the bf16 MFMA (k_shared.hip): the three bf16 parts of
 // rows of x ([S][K/32][3][32]); h = silu(Wg x) * (Wu x) as its parts; out = Wd h (f32)
 int sw_launch_sh_parts(hipStream_t st, const float *x, int S, int K, uint16_t *parts);
+// a transfer between this library's pinned staging and device scratch, in stream order (k_xfer.hip)
+hipError_t sw_xfer(hipStream_t st, void *dst, const void *src, size_t bytes, hipMemcpyKind kind);
 int sw_launch_sh_glu(hipStream_t st, const uint16_t *Wg, const uint16_t *Wu, const uint16_t *xp, int S, int D, int Is,
                      uint16_t *hp);
 int sw_launch_sh_down(hipStream_t st, const uint16_t *Wd, const uint16_t *hp, int S, int Is, int D, float *out);
