@@ -399,7 +399,9 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
                 __builtin_amdgcn_sched_barrier(0);
                 // (float)acc exactly, times s, times the token's power of two: dot8's
                 // (float)acc * (s * xf) with its one rounding, the second of a pair scaled by
-                // the fma that adds it
+                // the fma that adds it.  The bits are dot8's while s * xf and the terms are normal
+                // numbers; below (every input of a group under about 1e-29 at s = 1e-3) dot8's
+                // s * xf rounds to a denormal and this stays the nearer of the two
                 sw_f32x4 u;
 #pragma unroll
                 for (int j = 0; j < 4; j++) u[j] = __builtin_fmaf(R[i & 1][1][j], 4096.0f, R[i & 1][0][j]);
