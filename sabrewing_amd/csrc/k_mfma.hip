@@ -37,14 +37,19 @@
 // tile runs the loop of its own column count.
 //
 // What bounds it: the SIMDs' issue.  A step is 2 MFMAs, 4 conversions (one fma each), 4
-// products with s, 4 scalings (products or fmas with the power of two, exact) and 1-2 sums;
-// alone in registers, with two waves per SIMD, that takes 67 cycles -- MFMA and VALU time
-// add up -- against 130-160 here with the expansion (9 operations per 8 weights), LDS and
-// barriers.  LDS reads are 1 KB per step for two row tiles.  16 tokens (NT = 1) fit 128
-// registers, four waves per SIMD; 64 take 256, two.  Expanding in every wave from registers
-// replaced weights expanded once per block into LDS, whose reads (1 KB per row tile and
-// group) and barriers (one per chunk over 16 waves) bounded the loop: C2 S = 2048 gate_up
-// 1,676 -> 1,440 us, down 901 -> 776; S = 181 586 -> 447 and 320 -> 272.
+// products of scale and factor, 4 terms, 4 sums on average, and its share of the expansion
+// (9 operations per 8 weights): a quad of 4, 3, 2 or 1 columns has 603, 483, 363 or 247 VALU
+// instructions beside 64, 48, 32 or 16 MFMAs.  LDS reads are 1 KB per step for two row tiles.
+// Every term is rounded before it is added: a form that scaled acc by s and let the fma of the
+// add apply the power of two had 8 instructions fewer per quad, row tile and column and took
+// 3 % less at 64 tokens (C2 S = 2048 gate_up 1,456 against 1,505 us, S = 181 412 against 414), but left
+// dot8's bits where s * xf is no normal number, acc * s overflows or a term does.  16 tokens
+// (NT = 1) fit 128 registers, four waves per SIMD; 64 take 256, two, and spill: gate_up 22, down
+// 56 registers (group scales of 32), paid per run and row block but for one reload a quad.
+// Expanding in every wave from registers replaced weights expanded once per block into LDS,
+// whose reads (1 KB per row tile and group) and barriers (one per chunk over 16 waves) bounded
+// the loop: C2 S = 2048 gate_up 1,783 -> 1,505 us, down 990 -> 862; S = 181 571 -> 414 and
+// 314 -> 235; C1 S = 333 gate_up 148 -> 140, down 78 -> 82.
 #include "sw_hip.h"
 #include "sw_gate.h"
 
@@ -397,20 +402,15 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
                 const sw_f32x4 xf = op[(i >> 1) & 1].xf;
                 if (i + 1 < NS) mul(i + 1, op[((i + 1) >> 1) & 1], R[(i + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
-                // (float)acc exactly, times s, times the token's power of two: dot8's
-                // (float)acc * (s * xf) with its one rounding, the second of a pair scaled by
-                // the fma that adds it.  The bits are dot8's while s * xf and the terms are normal
-                // numbers; below (every input of a group under about 1e-29 at s = 1e-3) dot8's
-                // s * xf rounds to a denormal and this stays the nearer of the two
-                sw_f32x4 u;
-#pragma unroll
-                for (int j = 0; j < 4; j++) u[j] = __builtin_fmaf(R[i & 1][1][j], 4096.0f, R[i & 1][0][j]);
-                if constexpr (SM) u = u * sc[t][g];
+                // dot8's terms and sums: (float)acc, exact, times the product of s and the
+                // token's power of two
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    if (g == 0 || g == 2) h[t][j] = u[j] * xf[j];
-                    else if (g == 1) q[t][j] = __builtin_fmaf(u[j], xf[j], h[t][j]);
-                    else q[t][j] = q[t][j] + __builtin_fmaf(u[j], xf[j], h[t][j]);
+                    const float a_ = __builtin_fmaf(R[i & 1][1][j], 4096.0f, R[i & 1][0][j]);
+                    const float p = a_ * (SM ? sc[t][g] * xf[j] : xf[j]);
+                    if (g == 0 || g == 2) h[t][j] = p;
+                    else if (g == 1) q[t][j] = h[t][j] + p;
+                    else q[t][j] = q[t][j] + (h[t][j] + p);
                 }
                 // (formed here: the compiler would sink the sums to their last use, with every
                 // product live until then)

@@ -171,15 +171,19 @@ __host__ __device__ inline int sw_npass_max(int T, int E, int tt) { return (T + 
 #define SW_MF_TT 64               // the prefill MFMA kernels' largest token tile
 // The MFMA against dot8 for T packed rows in G groups: from 4.75 rows a group.  dot8's time
 // grows with the rows (24 dots per weight group and row), the MFMA's hardly does up to 16.
-// Measured per layer step, dot8 against the MFMA: C2 at 4.4 rows a group 693 / 720 us, at 5
-// 771 / 730, at 7 1,117 / 837; C1 at 4 114 / 126, at 6 142 / 120; D = 2048, I = 512, E = 256
-// at 4 209 / 193; C5 at 4 900 / 892.
+// The two cross between 3.5 and 4.5 rows, by half a row differently from run to run; the line
+// lies above that.  Per layer step, dot8 against the MFMA: C2 at 3.5 rows a group 617 / 678 us,
+// at 4.4 725 / 694, at 5 778 / 704, at 7 1,049 / 745; C1 at 4 108 / 103, at 6 139 / 106;
+// D = 2048, I = 512, E = 256 at 4 211 / 196; C5 at 4 909 / 901, at 4.75 1,030 / 926.
 __host__ __device__ inline bool sw_mf_wins(int64_t T, int64_t G) { return 4 * T >= 19 * G; }
 // tokens per tile of the MFMA launches: 16 (four waves per SIMD) up to 9 rows a group, 32 up
-// to 22, else 64 (each weight expanded once for four columns of tokens).  Measured per layer
-// step with 16 / 32 / 64: C2 at 5 rows a group 730 / 752 / 837 us, at 10 899 / 890 / 1,016, at
-// 27 1,485 / 1,249 / 1,256, at 40 1,903 / 1,700 / 1,473; C1 at 20 182 / 147 / 160, at 31
-// 225 / 206 / 180; C5 at 22 1,636 / 1,374 / 1,393
+// to 22, else 64 (each weight expanded once for four columns of tokens).  Per layer step with
+// 16 / 32 / 64: C2 at 5 rows a group 704 / 722 / 804 us, at 9 829 / 822 / 936, at 10 848 / 821
+// / 951, at 20 1,248 / 1,119 / 1,110, at 27 1,440 / 1,242 / 1,211, at 40 1,889 / 1,722 / 1,460;
+// C1 at 20 181 / 145 / 152, at 25 212 / 201 / 167; C5 at 22 1,667 / 1,439 / 1,433.  Those have
+// 64 groups or more.  The rule does not look at the grid: few groups in wide tiles leave CUs
+// idle (4 GLM experts of D = 5120, I = 1536, whole calls: 32 rows each 314 / 346 / 349 us, 64
+// rows 535 / 558 / 615; 16 experts of 64 rows 2,125 / 2,082 / 2,071).
 __host__ __device__ inline int sw_mf_cols(int64_t T, int64_t G) { return T <= 9 * G ? 16 : T <= 22 * G ? 32 : SW_MF_TT; }
 // the MFMA tiles of a group of n tokens, at most tt each: ceil(n / tt) of them, each of the
 // same whole number of 16-token columns (80 tokens in 64s: 48 + 32, not 64 + 16 -- a tail
