@@ -394,10 +394,12 @@ static void launch_lanes_w(hipStream_t st, const LanesArgs &A) {
               lds, st, A);
 }
 // whole 16-byte pieces: rows of W and of x at 16-byte strides and addresses, at least one
-// chain step in a row
+// chain step in a row; passes of 8 tokens within a grid's second dimension (k_lanes16's of 16
+// reach twice as far)
+#define LN_GRID_Y 65535
 static bool lanes_w_ok(const LanesArgs &A, int bits) {
-    return (size_t)A.I * bits / 8 % 16 == 0 && (size_t)A.I * bits % 8 == 0 && ((uintptr_t)A.W & 15) == 0 &&
-           ((uintptr_t)A.x & 15) == 0 && A.ldx % 4 == 0 && A.I >= 32;
+    return A.S <= 8 * LN_GRID_Y && (size_t)A.I * bits / 8 % 16 == 0 && (size_t)A.I * bits % 8 == 0 &&
+           ((uintptr_t)A.W & 15) == 0 && ((uintptr_t)A.x & 15) == 0 && A.ldx % 4 == 0 && A.I >= 32;
 }
 
 template <int WK, int DP>

@@ -78,3 +78,18 @@ def test_q4(be, orc, I, O):
             assert np.array_equal(bits(got), bits(orc.matmul_q4(x, p, sc))), (S, I, O)
     for b in (d0, d1, ds):
         b.free()
+
+
+@pytest.mark.parametrize("S", [8 * 65535, 8 * 65535 + 1])
+def test_most_tokens(be, orc, S):
+    """the last row count whose passes of 8 fit a grid's second dimension (65535), and one
+    more, which the general kernel's passes of 16 take"""
+    I = 32
+    rng = np.random.default_rng(S)
+    q = rng.integers(-127, 128, (1, I)).astype(np.int8)
+    sc = rng.uniform(1e-3, 2e-3, 1).astype(np.float32)
+    x = rng.standard_normal((S, I), dtype=np.float32)
+    dq, ds = be.upload(q), be.upload(sc)
+    got = be.matmul_q8(x, dq, ds, 1)
+    dq.free(); ds.free()
+    assert np.array_equal(bits(got), bits(orc.matmul_q8(x, q, sc, 0)))
