@@ -55,8 +55,8 @@ def test_nibble_kat(be):
 @pytest.mark.parametrize("S_", [1, 4, 40, 64, 65, 130])
 def test_matmul_bf16(be, orc, S_):
     """every row count reproduces the CPU's 16-lane f32-activation contract bit for
-    bit (the 16-lane kernel takes up to 16 tokens per weight pass, so 65 and 130 rows
-    run several passes), |x| up to 1e5 and tiny values included"""
+    bit (256 outputs: one token per weight pass up to 40 rows, two at 64 and 65, four at
+    130), |x| up to 1e5 and tiny values included"""
     O, I = 256, 1024
     rng = np.random.default_rng(3)
     Wb = orc.to_bf16((rng.standard_normal((O, I)) * 0.02).astype(np.float32))

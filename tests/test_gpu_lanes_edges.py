@@ -1,9 +1,10 @@
 """The host-activation matmuls where their two kernels meet (k_lanes.hip): rows in whole
 16-byte pieces are streamed by waves, everything else takes the general tiles.  Inputs around
 a step (128, 256 or 512 columns by the weight type), an x chunk (512 columns) and the scalar
-tail, outputs around a wave's 4 rows and a block's 16, tokens around the passes of 1, 2, 4 and
-8; a weight address off by one element takes the general kernel.  All bit for bit the
-oracle's, whose matmuls are pinned to the compiled reference."""
+tail, outputs around a wave's 4 rows and a block's 16; a weight address off by one element
+takes the general kernel.  With few outputs the streamed kernel runs a token at a time,
+whatever the batch; test_widths has enough of them for its passes of 1, 2, 4 and 8.  All bit
+for bit the oracle's, whose matmuls are pinned to the compiled reference."""
 import numpy as np
 import pytest
 
@@ -78,6 +79,46 @@ def test_q4(be, orc, I, O):
             assert np.array_equal(bits(got), bits(orc.matmul_q4(x, p, sc))), (S, I, O)
     for b in (d0, d1, ds):
         b.free()
+
+
+def _width(O, S):
+    """tokens per pass of the streamed kernel: the most that leave 512 blocks"""
+    ts = 8 if S >= 8 else 4 if S >= 3 else S
+    while ts > 1 and -(-O // 16) * -(-S // ts) < 512:
+        ts //= 2
+    return ts
+
+
+WIDE_O = 8195                                         # 513 blocks a pass: every width is reached
+WIDE_S = [1, 2, 3, 4, 7, 8, 9, 17]                    # full passes, and passes with tokens past the batch
+
+
+@pytest.mark.parametrize("kind,I", [("bf16", 32), ("bf16", 160), ("bf16", 536), ("bf16", 1056),
+                                    ("bf16_rx", 32), ("bf16_rx", 160), ("bf16_rx", 544), ("bf16_rx", 1056),
+                                    ("q8", 32), ("q8", 272), ("q8", 528), ("q8", 1040),
+                                    ("q4", 32), ("q4", 160), ("q4", 544), ("q4", 1056)])
+def test_widths(be, orc, kind, I):
+    """each width of the streamed kernel on full and partial steps and chunks"""
+    O = WIDE_O
+    assert [_width(O, S) for S in WIDE_S] == [1, 2, 4, 4, 4, 8, 8, 8]
+    rng = np.random.default_rng(I * 149 + len(kind))
+    sc = rng.uniform(1e-3, 2e-3, O).astype(np.float32)
+    if kind == "q8":
+        W = rng.integers(-127, 128, (O, I)).astype(np.int8)
+    elif kind == "q4":
+        W = rng.integers(0, 256, (O, I // 2), dtype=np.uint8)
+    else:
+        W = orc.to_bf16(rng.standard_normal((O, I)).astype(np.float32) * np.float32(0.02)).reshape(O, I)
+        W[0, :3] = [1, 0x8001, 0x7F]
+    d, ds = be.upload(W), be.upload(sc)
+    run, ref = {"bf16": (lambda x: be.matmul_bf16(x, d, O), lambda x: orc.matmul_bf16(x, W)),
+                "bf16_rx": (lambda x: be.matmul_bf16_rx(x, d, O), lambda x: orc.matmul_bf16_rx(x, W)),
+                "q8": (lambda x: be.matmul_q8(x, d, ds, O), lambda x: orc.matmul_q8(x, W, sc, 0)),
+                "q4": (lambda x: be.matmul_q4(x, d, ds, O, 0), lambda x: orc.matmul_q4(x, W, sc))}[kind]
+    for S in WIDE_S:
+        x = _x(rng, S, I)
+        assert np.array_equal(bits(run(x)), bits(ref(x))), S
+    d.free(); ds.free()
 
 
 @pytest.mark.parametrize("S", [8 * 65535, 8 * 65535 + 1])
