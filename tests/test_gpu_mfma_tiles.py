@@ -16,10 +16,10 @@ class _Layer:
     pass
 
 
-def _run(be, L, x, sizes, K, gs):
-    """group g: expert g, sizes[g] rows; every row is its own token (K = 1)"""
+def _run(be, L, x, sizes, K, gs, E=None):
+    """group g: expert g (mod E), sizes[g] rows; every row is its own token (K = 1)"""
     T = sum(sizes)
-    gexp, gcnt = np.arange(len(sizes), dtype=np.int32), np.array(sizes, np.int32)
+    gexp, gcnt = np.arange(len(sizes), dtype=np.int32) % (E or len(sizes)), np.array(sizes, np.int32)
     gbeg = np.concatenate([[0], np.cumsum(gcnt)[:-1]]).astype(np.int32)
     perm = np.random.default_rng(7).permutation(T).astype(np.int32)      # packed row -> token
     rowof = np.empty(T, np.int32)
@@ -53,4 +53,53 @@ def test_mfma_tiles_equal_dot8(be: Backend, gs, D, I, sizes):
     for b in (L.gu_q, L.gu_s, L.dn_q, L.dn_s):
         b.free()
     assert np.isfinite(out[DOT8]).all()
+    assert np.array_equal(out[MFMA].view(np.uint32), out[DOT8].view(np.uint32))
+
+
+def _tile_width(sizes):
+    T, G = sum(sizes), len(sizes)
+    return 16 if T <= 9 * G else 32 if T <= 22 * G else 64
+
+
+def _row_blocks(D, sizes):
+    """the down's row blocks per block: up to four while that leaves 1024 blocks"""
+    tt, nrb = _tile_width(sizes), -(-D // 256)
+    tiles = sum(-(-n // tt) for n in sizes)
+    return next((r for r in (4, 2) if nrb % r == 0 and tiles * (nrb // r) >= 1024), 1)
+
+
+# (D, groups, rows per group, tile width, row blocks per block): D of 3.5 and 7.5 row blocks
+MANY = [(1920, 600, (1, 9), 16, 4), (1920, 300, (1, 9), 16, 2), (1920, 560, (8, 23), 32, 4), (1920, 300, (8, 23), 32, 2),
+        (1920, 520, (17, 33), 64, 4), (1920, 260, (17, 60), 64, 2), (896, 1000, (1, 22), 32, 2), (896, 1000, (1, 16), 16, 4)]
+
+
+@pytest.mark.parametrize("gs", [0, 32])
+@pytest.mark.parametrize("I", [128, 384, 512])
+@pytest.mark.parametrize("D,G,lohi,tt,r", MANY, ids=lambda v: str(v).replace(" ", ""))
+def test_down_over_several_row_blocks(be: Backend, D, G, lohi, tt, r, I, gs):
+    """many groups: a down block runs 2 or 4 row blocks through one pipeline (the digits of a
+    chunk again for each, the next row block's weights ahead), with 1, 3 and 4 quads of inputs
+    (a half-filled last chunk where a chunk holds two) and outputs that end in half a row block"""
+    rng = np.random.default_rng(D + I + G)
+    sizes = [int(n) for n in rng.integers(*lohi, G)]
+    if (tt, r) == (16, 4) and D == 896:
+        sizes[:40] = [17] * 40                        # (two tiles each: beyond 1024 tiles)
+    assert (_tile_width(sizes), _row_blocks(D, sizes)) == (tt, r)
+    E, n = 4, lambda K: K // gs if gs else 1
+    L = _Layer()
+    L.D, L.I = D, I
+    q = lambda rows, K: be.upload(rng.integers(0, 256, (rows, K // 2), dtype=np.uint8))
+    s = lambda rows, K: be.upload(rng.uniform(1e-3, 4e-3, (rows, n(K))).astype(np.float32))
+    L.gu_q, L.gu_s, L.dn_q, L.dn_s = q(E * 2 * I, D), s(E * 2 * I, D), q(E * D, I), s(E * D, I)
+    x = rng.standard_normal((sum(sizes), D), dtype=np.float32)
+    out = {}
+    for mode in (DOT8, MFMA):
+        prev = be.set_grouped_kernel(mode)
+        try:
+            out[mode] = _run(be, L, x, sizes, 1, gs, E)
+        finally:
+            be.set_grouped_kernel(prev)
+    for b in (L.gu_q, L.gu_s, L.dn_q, L.dn_s):
+        b.free()
+    assert np.isfinite(out[DOT8]).all() and (out[DOT8] != 0).any()
     assert np.array_equal(out[MFMA].view(np.uint32), out[DOT8].view(np.uint32))
