@@ -507,7 +507,7 @@ static int mf_go(hipStream_t st, unsigned nblocks, const MfArgs &A) {
 }
 template <int GLU, int PT = 0>
 static int mf_dispatch(hipStream_t st, unsigned nblocks, const MfArgs &A) {
-    const int tt = A.grp.tt ? A.grp.tt : SW_MF_TT;
+    const int tt = A.grp.tt;
 #define SW_MF_SM(N_) \
     (A.W.gs <= 0 ? mf_go<GLU, N_, 0, PT>(st, nblocks, A) \
      : A.W.gs == SW_RG ? mf_go<GLU, N_, 1, PT>(st, nblocks, A) \

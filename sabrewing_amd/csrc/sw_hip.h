@@ -144,10 +144,11 @@ struct SwGroups {
     int ngroups_max;                 // grid extent: groups, or passes when items is set
     int cnt_const;
     // passes (optional): items[j] = (t0 << 10) | group of pass j, P = the device count;
-    // a block then takes one pass of up to DG_TT tokens from t0 instead of a whole group
+    // a block then takes one pass of up to tt tokens from t0 instead of a whole group; the
+    // step between a group's passes follows from tt, so it must be the listing's
     const int *items;
     const int *P;
-    int tt;                          // tokens per pass of the items (1 or 2; 0: SW_DG_TT)
+    int tt;                          // the tokens per pass the items were listed with: dot8 1 or 2 (0: SW_DG_TT), MFMA 16, 32 or 64
 };
 #define SW_DG_TT 2             // tokens per weight pass of the grouped dot8 kernels
 // route activations whose gate is a softmax of the logits (computed with the
@@ -168,7 +169,7 @@ __host__ __device__ inline bool sw_act_scores(int act) { return act == 0 || act 
 struct SwGateOpt { int ld, ns; float rs; int wld; float *wsh; int wshld; };
 // the upper bound of the passes of T packed rows in at most min(T, E) groups, tt tokens each
 __host__ __device__ inline int sw_npass_max(int T, int E, int tt) { return (T + (T < E ? T : E) * (tt - 1)) / tt; }
-#define SW_MF_TT 64               // the prefill MFMA kernels' largest token tile
+#define SW_MF_TT 64               // the MFMA kernels' largest token tile
 // The MFMA against dot8 for T packed rows in G groups: from 4.75 rows a group.  dot8's time
 // grows with the rows (24 dots per weight group and row), the MFMA's hardly does up to 16.
 // The two cross between 3.5 and 4.5 rows, by half a row differently from run to run; the line
@@ -376,8 +377,8 @@ int sw_launch_stage_experts(hipStream_t st, SwQ4 W, const sw_u32x4 *xl, const fl
 // stack glue (k_glue.hip): RMSNorm rows, greedy argmax rows
 // prefill expert GEMMs on the f16 MFMA (k_mfma.hip), bit-identical to the
 // dot8 ones: activations as MFMA digits dg[rows][K/32][32 dwords] + factors
-// xs[rows][K/32] (the limbs' exponent and integer, recut); tiles of up to 64
-// tokens of a group listed in g.items / g.P (sw_launch_bucket with tt = SW_MF_TT)
+// xs[rows][K/32] (the limbs' exponent and integer, recut); tiles of up to g.tt = 16, 32 or
+// 64 tokens of a group (any other is refused) listed in g.items / g.P with the same tt
 #define SW_MF_DIGIT_BYTES 128     // MFMA digits of one (row, input group): 32 dwords
 int sw_launch_digits(hipStream_t st, const float *x, int rows, int K, uint32_t *dg, float *xs);
 // (dg_rows: the rows of dg and xs; dg_rows * K * 4 must stay below 2^32)
