@@ -171,8 +171,10 @@ GLay glay(const Groups &G, int T, int xrows, int nextra = 0, bool mf = false) {
     L.end = cv.off;
     return L;
 }
-// the f16 MFMA GEMMs from 8 rows a group on (the lag family's groups are many, and take them
-// from fewer): whole quads of 4 input groups
+// the f16 MFMA GEMMs from 8 rows a group on: whole quads of 4 input groups.  At 8 rows they are
+// well ahead, and the two cross below (dot8 / MFMA, whole calls, D = 5120, I = 1536: 4 experts
+// of 4 rows 100 / 114 us, 5 rows 122 / 122, 8 rows 174 / 142; 8 experts of 3 rows 129 / 129, 5
+// rows 191 / 157, 8 rows 299 / 216; 16 experts of 2 rows 147 / 158, 3 rows 206 / 182)
 bool use_mf(const Groups &G) { return G.D % 128 == 0 && G.I % 128 == 0 && G.total >= 8 * G.count; }
 // the ints and the table in the host image H of the scratch's head: gexp = 0..count-1 (the
 // table index), gbeg, gcnt, n further ints (grow, or the MFMA tiles); the table

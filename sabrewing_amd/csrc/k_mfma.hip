@@ -17,11 +17,11 @@
 // operations one for one, so a token's output has the same bits whichever
 // kernel ran its group.
 //
-// Digits in memory: per (input row, group) 128 bytes, E0 of the 32 inputs as
-// f16, then E1: the B operands of the two MFMAs.  Lane l of an MFMA (column
-// l % 16, k quarter q = l / 16) reads the 16 bytes of inputs 8q .. 8q+7 (in
-// the slot order of mf_expand), and its A operand holds the same inputs of a
-// weight row as f16, expanded from packed dword q of the row's group.
+// Digits in memory: per (input row, group) 128 bytes, E0 of the 32 inputs as f16, then E1: the
+// A operands of the two MFMAs (A rows: tokens; B columns: weight rows).  Lane l of an MFMA
+// (token, resp. weight row, l % 16; k quarter q = l / 16) reads the 16 bytes of inputs 8q ..
+// 8q+7 of its token (in the slot order of mf_expand), and its B operand holds the same inputs
+// of its weight row as f16, expanded from packed dword q of the row's group.
 //
 // Block: 256 weight rows x a tile of up to 16 NT tokens (NT columns of 16) of one group, 8
 // waves.  A wave owns two 16-row tiles (for gate_up the gate and the up rows of the same 16
@@ -29,9 +29,8 @@
 // of each of its rows straight into registers -- a lane the whole packed group kq of its row,
 // transposed within the lanes by permlane swaps -- expands each weight once for all the
 // tile's columns, and reads the columns' digits and factors from LDS, where the block stages
-// them in two buffers, a chunk of quads ahead.  The MFMA takes the digits as its A (rows:
-// tokens) and the weights as its B (columns: weight rows), so a lane's four results are of
-// one weight row, whose scale is a plain register, and of four tokens.  Loads of a quad are
+// them in two buffers, a chunk of quads ahead.  A lane's four results are of one weight row,
+// whose scale is a plain register, and of four tokens.  Loads of a quad are
 // issued a quad ahead, a step's two MFMAs one step (column, group, row tile) ahead of its
 // sums.  A group's tokens are split into equal tiles of whole columns (sw_mf_tile), and a
 // tile runs the loop of its own column count.
@@ -165,12 +164,6 @@ __device__ __forceinline__ void mf_transpose(const sw_u32x4 &r, uint32_t (&o)[4]
     o[0] = c.x; o[1] = c.y; o[2] = d.x; o[3] = d.y;
 }
 
-// the value of lane J of each lane's quad (DPP quad_perm [J, J, J, J])
-template <int J>
-__device__ __forceinline__ float mf_quad_bcast(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x55 * J, 0xF, 0xF, true));
-}
-
 // NT: the tile's most 16-token columns; SM: the weight scales, 0 one per row (after the
 // sum), 1 one per 32 inputs, 2 one per 64, 3 one per 128 or more (one a quad)
 template <int GLU, int NT, int SM, int PT>
@@ -230,8 +223,8 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
         return eo + (uint32_t)(min(rb * RPB + lr, O - 32) + 16 * t);
     };
     struct Raw { sw_u32x4 q[2]; sw_f32x4 s[2]; };
-    // quad c of row block rb: 64 bytes of each of the tile's 16 rows, and lane col & 3's
-    // scales of row 4 kq + (col & 3) (moved to the quad's products by DPP)
+    // quad c of row block rb: 64 bytes of each of the tile's 16 rows, 16 per lane, and the quad's
+    // four scales of the lane's own row col (the same in the row's four lanes)
     auto load_w = [&](Raw &R, int rb, int c) {
         const uint32_t cu = (uint32_t)__builtin_amdgcn_readfirstlane(c);
 #pragma unroll
@@ -540,9 +533,8 @@ int sw_launch_mf_glu(hipStream_t st, SwQ4 W, const uint32_t *dg, const float *xs
     int gsh;
     if (mf_check(W, g, gsh, dg_rows) || I % 128 || W.O != 2 * I) return -1;
     const int nrb = I / 128;
-    const int rp = 1;
-    const MfArgs A = {W, gsh, dg, xs, dg_rows, g, I, nrb, rp, hdg, hxs, nullptr};
-    return mf_dispatch<1>(st, (unsigned)(g.ngroups_max * (nrb / rp)), A);
+    const MfArgs A = {W, gsh, dg, xs, dg_rows, g, I, nrb, 1, hdg, hxs, nullptr};
+    return mf_dispatch<1>(st, (unsigned)(g.ngroups_max * nrb), A);
 }
 
 int sw_launch_mf_rows(hipStream_t st, SwQ4 W, const uint32_t *dg, const float *xs, int dg_rows, SwGroups g, float *Y) {
@@ -562,9 +554,8 @@ int sw_launch_mf_glu_tab(hipStream_t st, SwQ4 W, const SwTab *tab, const uint32_
     W.E = 1;
     if (!tab || !hdg || !hxs || mf_check(W, g, gsh, dg_rows) || I % 128 || W.O != 2 * I) return -1;
     const int nrb = I / 128;
-    const int rp = 1;
-    const MfArgs A = {W, gsh, dg, xs, dg_rows, g, I, nrb, rp, hdg, hxs, nullptr, tab};
-    return mf_dispatch<1, 1>(st, (unsigned)(g.ngroups_max * (nrb / rp)), A);
+    const MfArgs A = {W, gsh, dg, xs, dg_rows, g, I, nrb, 1, hdg, hxs, nullptr, tab};
+    return mf_dispatch<1, 1>(st, (unsigned)(g.ngroups_max * nrb), A);
 }
 int sw_launch_mf_rows_tab(hipStream_t st, SwQ4 W, const SwTab *tab, const uint32_t *dg, const float *xs, int dg_rows,
                           SwGroups g, float *Y) {

@@ -14,7 +14,7 @@ __global__ __launch_bounds__(256) void k_xfer(void *__restrict__ dst, const void
 // 5 us a transfer from 64 KB or so on (below, the runtime copies by a kernel of its own); a
 // kernel is ordered by the stream.  Beyond some 1 MB the engine's rate over the link is worth
 // more.  Whole calls, engine / kernel: a bf16 matmul of 4096 x 4096, 2 tokens (32 KB each
-// way) 45 / 34 us, 16 (256 KB) 81 / 71, 64 (1 MB) 206 / 202; a 8-expert int4 group of one row
+// way) 45 / 34 us, 16 (256 KB) 81 / 71, 64 (1 MB) 206 / 202; an 8-expert int4 group of one row
 // each (160 KB) 81 / 70; groups of 96 rows (1.9 MB) 318 / 323, of 256 (5 MB) 1,074 / 1,174.
 #define XFER_KERNEL_MAX ((size_t)1 << 20)
 hipError_t sw_xfer(hipStream_t st, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
