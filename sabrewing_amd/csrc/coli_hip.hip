@@ -7,7 +7,7 @@
 // sticky error consumed (c/backend_cuda.cu:63-69), COLI_GPU_FAIL_AFTER=N
 // failing every compute entry after N calls (c/backend_cuda.cu:667-677).
 //
-// Different inside: a whole expert group is four launches whatever its count
+// Different inside: a whole expert group is three kernels whatever its count
 // (limbs of x, gate/up + SiLU-GLU over every group, down over every group),
 // the int4 bytes stay as stored (the signed-nibble XOR happens in registers),
 // and each group reads its three tensors through a per-group table, so the
@@ -185,7 +185,7 @@ void pack_meta(const Groups &G, const GLay &L, const int *more, int n, char *H) 
     memcpy(H + L.tab, G.tab.data(), (size_t)G.count * sizeof(SwTab));
 }
 
-// the four launches: limbs of xrows rows, gate/up + GLU, down -> y [T][D]
+// the three launches: limbs of xrows rows, gate/up + GLU, down -> y [T][D]
 int launch_group(Ctx *c, const Groups &G, char *A, const GLay &L, int T, int xrows, bool with_grow) {
     const int *d = (const int *)(A + L.ints);
     const SwTab *tab = (const SwTab *)(A + L.tab);

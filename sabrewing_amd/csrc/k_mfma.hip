@@ -35,16 +35,19 @@
 // sums.  A group's tokens are split into equal tiles of whole columns (sw_mf_tile), and a
 // tile runs the loop of its own column count.
 //
-// What bounds it: the SIMDs' issue.  A step is 2 MFMAs, 4 conversions (one fma each), 4
-// products of scale and factor, 4 terms, 4 sums on average, and its share of the expansion
-// (9 operations per 8 weights): a quad of 4, 3, 2 or 1 columns has 603, 483, 363 or 247 VALU
-// instructions beside 64, 48, 32 or 16 MFMAs.  LDS reads are 1 KB per step for two row tiles.
-// Every term is rounded before it is added: a form that scaled acc by s and let the fma of the
-// add apply the power of two had 8 instructions fewer per quad, row tile and column and took
-// 3 % less at 64 tokens (C2 S = 2048 gate_up 1,456 against 1,505 us, S = 181 412 against 414), but left
-// dot8's bits where s * xf is no normal number, acc * s overflows or a term does.  16 tokens
-// (NT = 1) fit 128 registers, four waves per SIMD; 64 take 256, two, and spill: gate_up 22, down
-// 56 registers (group scales of 32), paid per run and row block but for one reload a quad.
+// What bounds it: no one unit.  A step is 2 MFMAs, 4 conversions (one fma each), 4 products of
+// scale and factor, 4 terms, 4 sums on average, and its share of the expansion (9 operations
+// per 8 weights): a quad of 4, 3, 2 or 1 columns has 603, 483, 363 or 247 VALU instructions
+// beside 64, 48, 32 or 16 MFMAs.  VALU issue is the largest part, but 12 % more instructions
+// in the loop took 3 % longer at 64 tokens and 7 % more 0.6-1.5 % at 16; at 64 tokens the
+// waves, two per SIMD, spend 25-30 % of their time waiting (LDS reads, 1 KB per step for two
+// row tiles, and a barrier per chunk).  (Those instructions round every term before it is added.  Acc
+// times s, with the power of two applied by the fma of the add, had 8 fewer per quad, row tile
+// and column: C2 S = 2048 gate_up 1,456 against 1,505 us, S = 181 412 against 414.  It left
+// dot8's bits where s * xf is no normal number, acc * s overflows or a term does.)
+// 16 tokens (NT = 1) fit 128 registers, four waves per SIMD; 64 take 256, two, and spill:
+// gate_up 22, down 56 registers (group scales of 32), paid per run and row block but for one
+// reload a quad.
 // Expanding in every wave from registers replaced weights expanded once per block into LDS,
 // whose reads (1 KB per row tile and group) and barriers (one per chunk over 16 waves) bounded
 // the loop: C2 S = 2048 gate_up 1,783 -> 1,505 us, down 990 -> 862; S = 181 571 -> 414 and
