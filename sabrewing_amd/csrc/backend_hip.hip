@@ -260,7 +260,7 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
     if (D <= 0 || I <= 0 || G <= 0 || S <= 0) return -1;
     const int T = S * K;
     // the MFMA kernels for prefill-sized groups: tiles of up to tt tokens, listed here
-    const int tt = sw_mf_cols(T, G);
+    const int tt = sw_mf_cols(T, G, D, I);
     int ntile = 0;
     for (int i = 0; i < G; i++) ntile += (gcnt[i] + tt - 1) / tt;
     const bool mf = G < 1024 && T < (1 << 21) && use_mfma(T, G, D, I);
@@ -778,7 +778,7 @@ static int forward(const LagHipMoeDesc *d, const LagHipMoeWeights *w, const floa
               return fail_msg("down/combine launch"); }
         g_last_G_dev = 0; g_last_ng = K;
     } else if (mf) {                     // prefill: tiles of up to 64 tokens of a group on the f16 MFMA
-        const int tt = sw_mf_cols(T, T < E ? T : E);
+        const int tt = sw_mf_cols(T, T < E ? T : E, D, I);
         { PROF("bucket");
           // (the split sort's counts in the slots, which the down launch writes later)
           if (sw_launch_bucket(g_st, f.sel, S, K, E, f.gexp, f.gbeg, f.gcnt, f.G, f.grow, f.rowof, tt, f.items, f.P,

@@ -181,11 +181,19 @@ __host__ __device__ inline bool sw_mf_wins(int64_t T, int64_t G) { return 4 * T 
 // to 22, else 64 (each weight expanded once for four columns of tokens).  Per layer step with
 // 16 / 32 / 64: C2 at 5 rows a group 704 / 722 / 804 us, at 9 829 / 822 / 936, at 10 848 / 821
 // / 951, at 20 1,248 / 1,119 / 1,110, at 27 1,440 / 1,242 / 1,211, at 40 1,889 / 1,722 / 1,460;
-// C1 at 20 181 / 145 / 152, at 25 212 / 201 / 167; C5 at 22 1,667 / 1,439 / 1,433.  Those have
-// 64 groups or more.  The rule does not look at the grid: few groups in wide tiles leave CUs
-// idle (4 GLM experts of D = 5120, I = 1536, whole calls: 32 rows each 314 / 346 / 349 us, 64
-// rows 535 / 558 / 615; 16 experts of 64 rows 2,125 / 2,082 / 2,071).
-__host__ __device__ inline int sw_mf_cols(int64_t T, int64_t G) { return T <= 9 * G ? 16 : T <= 22 * G ? 32 : SW_MF_TT; }
+// C1 at 20 181 / 145 / 152, at 25 212 / 201 / 167; C5 at 22 1,667 / 1,439 / 1,433.
+// Few blocks: a launch has tiles x I / 128 (gate_up) or D / 256 (down) blocks, and a
+// block alone on its CU takes 46 us with one column (gate_up, K = 4096), 66 with two, 85 with
+// three, 121 with four; so while a tile half as wide still gives every block a CU of its own,
+// it is taken: below 112 blocks of 256 CUs, not 128, for the groups that end in a partial tile.
+// gate_up + down with 16 / 32 / 64: D = 4096, I = 1024, a group of 64 rows 62 / 88 / 159 us, 4
+// of 64 78 / 92 / 164, 4 of 128 136 / 117 / 170; D = 5120, I = 1536, 4 of 64 86 / 106 / 165.
+inline int sw_mf_cols(int64_t T, int64_t G, int D, int I) {
+    int tt = T <= 9 * G ? 16 : T <= 22 * G ? 32 : SW_MF_TT;
+    const int64_t nb = I / 128 < (D + 255) / 256 ? I / 128 : (D + 255) / 256;
+    while (tt > 16 && (T > G * tt ? (T + tt - 1) / tt : G) * nb < 112) tt >>= 1;
+    return tt;
+}
 // the MFMA tiles of a group of n tokens, at most tt each: ceil(n / tt) of them, each of the
 // same whole number of 16-token columns (80 tokens in 64s: 48 + 32, not 64 + 16 -- a tail
 // column costs most of what a full tile's staging does)

@@ -20,6 +20,7 @@ import pytest
 from oracle import synth
 from sabrewing_amd import configs as cf
 from sabrewing_amd.coli import Coli, ColiError
+from test_gpu_mfma_tiles import tile_width
 
 pytestmark = pytest.mark.gpu
 
@@ -136,18 +137,25 @@ def test_expert_group_one_row_each(coli, be, orc, gs):
 
 
 @pytest.mark.parametrize("gs", [0, 32])
-def test_prefill_group_on_the_mfma(coli, be, orc, gs):
-    """groups averaging >= 8 rows take the f16 MFMA GEMMs (64-token tiles, partial tiles,
-    one group over two tiles): still each row's lag expert output bit for bit"""
+@pytest.mark.parametrize("ids,rows,tt", [([3, 1, 4, 0], [40, 70, 9, 130], 16),
+                                         ([3, 1, 4, 0, 5, 2] * 5, [12, 9, 32, 15, 17, 10] * 5, 32),
+                                         ([3, 1, 4, 0, 5, 2] * 5, [40, 70, 9, 130, 1, 64] * 5, 64)],
+                         ids=["tiles16", "tiles32", "tiles64"])
+def test_prefill_group_on_the_mfma(coli, be, orc, gs, ids, rows, tt):
+    """groups averaging >= 8 rows take the f16 MFMA GEMMs (partial tiles, groups over several
+    tiles; 16-token tiles for four groups, which are few blocks, 32- and 64-token tiles for
+    30): still each row's lag expert output bit for bit"""
+    assert tile_width(rows, D, I) == tt
     L = layer(orc, gs, seed=21)
     ex = Experts(coli, L, gs)
-    ids, rows = [3, 1, 4, 0], [40, 70, 9, 130]
     T = sum(rows)
     x = np.random.default_rng(7).standard_normal((T, D)).astype(np.float32)
     y = coli.expert_group(*ex.lists(ids), rows, x)
     dev = [be.upload(a) for a in (L.gu_q, L.gu_s, L.dn_q, L.dn_s)]
     owner = np.repeat(ids, rows)
-    for r in list(range(0, T, 7)) + [39, 40, 109, 110, 118, 119, 182, 183, T - 1]:
+    ends = np.cumsum(rows)
+    for r in sorted(set(range(0, T, 7 if T < 300 else 31)) | {int(v) - 1 for v in ends} | {int(v) for v in ends[:-1]} |
+                    {182, 183}):
         e = int(owner[r])
         assert np.array_equal(bits(y[r]), bits(lag_expert(be, dev, L, e, x[r], gs))), (e, r)
         if r % 35 == 0:

@@ -15,6 +15,7 @@ import pytest
 from oracle import synth
 from sabrewing_amd import configs as cf
 from sabrewing_amd.backend import DeviceLayer, desc_of
+from test_gpu_mfma_tiles import tile_width
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-3
@@ -63,12 +64,12 @@ def test_mfma_equals_dot8_small(be, orc, cfg, S_):
     assert errs(got_m, want, base) <= TOL
 
 
-def test_mfma_multi_tile_groups(be, orc):
-    """groups of 100-200 tokens: two to four 64-token tiles each, the last one
-    partial, and one group with exactly 64"""
-    cfg = cf.scaled(cf.C1, D=512, E=8, K=2, I=256, name="C1-E8")
+@pytest.mark.parametrize("E,K,S_", [(8, 2, 400), (32, 4, 1000)], ids=["tiles16", "tiles64"])
+def test_mfma_multi_tile_groups(be, orc, E, K, S_):
+    """groups of 100-200 tokens: several tiles each, the last ones partial; 16-token tiles
+    for eight groups, which are few blocks, and 64-token tiles for 32 groups"""
+    cfg = cf.scaled(cf.C1, D=512, E=E, K=K, I=256, name=f"C1-E{E}")
     L = synth.make_layer(orc, cfg, 61)
-    S_ = 400
     x = synth.make_x(orc, cfg, 62, S_)
     base = np.zeros_like(x)
     dl = DeviceLayer.from_host(be, cfg, L)
@@ -78,7 +79,7 @@ def test_mfma_multi_tile_groups(be, orc):
     # per-token (decode path) for a few streams
     single = np.stack([block(be, cfg, dl, x[s:s + 1], base[s:s + 1], AUTO)[0] for s in (0, 199, 399)])
     dl.free()
-    assert max(gcnt[:G]) > 64
+    assert max(gcnt[:G]) > 64 and tile_width([int(n) for n in gcnt[:G]], cfg.D, cfg.I) == (16 if E == 8 else 64)
     assert np.array_equal(bits(got_m), bits(got_d))
     assert np.array_equal(bits(got_m[[0, 199, 399]]), bits(single))
     assert errs(got_m, orc.moe_block_rows(synth.desc_of(cfg), L, x, base), base) <= TOL

@@ -8,9 +8,11 @@ import numpy as np
 import pytest
 
 from sabrewing_amd.backend import Backend
+from test_gpu_mfma_tiles import tile_width, wide
 
 pytestmark = pytest.mark.gpu
 DOT8, MFMA = 1, 2
+E = 5
 D, I = 1152, 384                    # 9 and 3 quads of input groups: a short last run each
 
 
@@ -81,7 +83,8 @@ def _run(be, b, x, sizes, gs):
     perm = np.random.default_rng(7).permutation(T).astype(np.int32)
     rowof = np.empty(T, np.int32)
     rowof[perm] = np.arange(T, dtype=np.int32)
-    return be.moe_group(x, L, np.arange(len(sizes), dtype=np.int32), gbeg, gcnt, perm, rowof, np.ones((T, 1), np.float32), 1, gs)
+    gexp = np.arange(len(sizes), dtype=np.int32) % E
+    return be.moe_group(x, L, gexp, gbeg, gcnt, perm, rowof, np.ones((T, 1), np.float32), 1, gs)
 
 
 def _equal(a, b):
@@ -90,10 +93,13 @@ def _equal(a, b):
 
 
 @pytest.mark.parametrize("gs", [0, 32, 64, 128])
-@pytest.mark.parametrize("sizes", [[1, 16, 2, 15, 3], [17, 16, 31, 1, 32], [33, 64, 63, 81, 5]], ids=["cols16", "cols32", "cols64"])
+@pytest.mark.parametrize("sizes,tt", [([1, 16, 2, 15, 3], 16), ([17, 16, 31, 1, 32], 32), ([33, 64, 63, 81, 5], 64)],
+                         ids=["cols16", "cols32", "cols64"])
 @pytest.mark.parametrize("kind", list(KINDS))
-def test_bits_outside_the_ordinary(be: Backend, kind, sizes, gs):
-    E, T = len(sizes), sum(sizes)
+def test_bits_outside_the_ordinary(be: Backend, kind, sizes, tt, gs):
+    sizes = wide(sizes, D, I)
+    assert tile_width(sizes, D, I) == tt
+    T = sum(sizes)
     rng = np.random.default_rng(gs + T)
     n = lambda K: K // gs if gs else 1
     q = lambda r, K: rng.integers(0, 256, (r, K // 2), dtype=np.uint8)

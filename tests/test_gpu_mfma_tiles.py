@@ -1,5 +1,6 @@
 """The MFMA GEMMs (k_mfma.hip) at the edges of their tiles, through lag_hip_moe_group: groups
-of every size around a column (16 tokens) and a tile (16, 32 or 64 by the average group),
+of every size around a column (16 tokens) and a tile (16, 32 or 64 tokens by the average group
+and the launch's blocks),
 inputs of 1, 2, 3 and 4 quads of groups and beyond a run, outputs that end in half a row
 block, every scale layout.  dot8 forms the same sums in the same order, so the bits must be
 equal; dot8 itself is checked against the oracle in test_gpu_moe.py."""
@@ -28,13 +29,32 @@ def _run(be, L, x, sizes, K, gs, E=None):
     return be.moe_group(x, L, gexp, gbeg, gcnt, perm, rowof, w, K, gs)
 
 
+def tile_width(sizes, D, I):
+    """the launch rule (sw_mf_cols): by the average group, narrower while few blocks leave CUs idle"""
+    T, G = sum(sizes), len(sizes)
+    tt = 16 if T <= 9 * G else 32 if T <= 22 * G else 64
+    while tt > 16 and max(G, -(-T // tt)) * min(I // 128, -(-D // 256)) < 112:
+        tt //= 2
+    return tt
+
+
+def wide(sizes, D, I):
+    """the groups repeated until their launch takes the widest tile their average allows"""
+    reps = -(-112 // (min(I // 128, -(-D // 256)) * len(sizes)))
+    return sizes * reps
+
+
 @pytest.mark.parametrize("gs", [0, 32, 64, 128])
 @pytest.mark.parametrize("D,I", [(128, 128), (256, 384), (384, 256), (640, 128), (1152, 512)])
-@pytest.mark.parametrize("sizes", [[1, 16, 2, 15, 3], [17, 16, 31, 1, 32], [33, 64, 63, 16, 5], [65, 129, 48, 1, 80]],
-                         ids=["cols16", "cols32", "cols64", "split"])
-def test_mfma_tiles_equal_dot8(be: Backend, gs, D, I, sizes):
+@pytest.mark.parametrize("sizes,tt", [([1, 16, 2, 15, 3], 16), ([17, 16, 31, 1, 32], 32), ([33, 64, 63, 16, 5], 64),
+                                      ([65, 129, 48, 1, 80], 64)], ids=["cols16", "cols32", "cols64", "split"])
+@pytest.mark.parametrize("many", [False, True], ids=["few", "many"])
+def test_mfma_tiles_equal_dot8(be: Backend, gs, D, I, sizes, tt, many):
     rng = np.random.default_rng(D + I + gs)
     E, n = len(sizes), lambda K: K // gs if gs else 1
+    if many:
+        sizes = wide(sizes, D, I)
+    assert tile_width(sizes, D, I) == (tt if many else 16)
     L = _Layer()
     L.D, L.I = D, I
     q = lambda r, K: be.upload(rng.integers(0, 256, (r, K // 2), dtype=np.uint8))
@@ -47,7 +67,7 @@ def test_mfma_tiles_equal_dot8(be: Backend, gs, D, I, sizes):
     for mode in (DOT8, MFMA):
         prev = be.set_grouped_kernel(mode)
         try:
-            out[mode] = _run(be, L, x, sizes, 1, gs)
+            out[mode] = _run(be, L, x, sizes, 1, gs, E)
         finally:
             be.set_grouped_kernel(prev)
     for b in (L.gu_q, L.gu_s, L.dn_q, L.dn_s):
@@ -56,14 +76,9 @@ def test_mfma_tiles_equal_dot8(be: Backend, gs, D, I, sizes):
     assert np.array_equal(out[MFMA].view(np.uint32), out[DOT8].view(np.uint32))
 
 
-def _tile_width(sizes):
-    T, G = sum(sizes), len(sizes)
-    return 16 if T <= 9 * G else 32 if T <= 22 * G else 64
-
-
-def _row_blocks(D, sizes):
+def _row_blocks(D, I, sizes):
     """the down's row blocks per block: up to four while that leaves 1024 blocks"""
-    tt, nrb = _tile_width(sizes), -(-D // 256)
+    tt, nrb = tile_width(sizes, D, I), -(-D // 256)
     tiles = sum(-(-n // tt) for n in sizes)
     return next((r for r in (4, 2) if nrb % r == 0 and tiles * (nrb // r) >= 1024), 1)
 
@@ -84,7 +99,7 @@ def test_down_over_several_row_blocks(be: Backend, D, G, lohi, tt, r, I, gs):
     sizes = [int(n) for n in rng.integers(*lohi, G)]
     if (tt, r) == (16, 4) and D == 896:
         sizes[:40] = [17] * 40                        # (two tiles each: beyond 1024 tiles)
-    assert (_tile_width(sizes), _row_blocks(D, sizes)) == (tt, r)
+    assert (tile_width(sizes, D, I), _row_blocks(D, I, sizes)) == (tt, r)
     E, n = 4, lambda K: K // gs if gs else 1
     L = _Layer()
     L.D, L.I = D, I
