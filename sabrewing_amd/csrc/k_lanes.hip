@@ -29,7 +29,7 @@
 // shape of the launch that computed it.
 //
 // k_lanes_w streams rows of whole 16-byte pieces (below).  k_lanes16 takes the rest -- the
-// group-scaled int4, odd row lengths, odd addresses: 256 threads = 16 rows x 16 lanes; tiles
+// group-scaled int4, odd row lengths, odd addresses, short rows of many blocks: 256 threads = 16 rows x 16 lanes; tiles
 // of CC columns of the 16 rows (coalesced 16-byte loads) and of up to TS tokens go through
 // LDS, and each token's chains stay in registers across tiles.
 #include "sw_hip.h"
@@ -401,11 +401,21 @@ static bool lanes_w_ok(const LanesArgs &A, int bits) {
     return A.S <= 8 * LN_GRID_Y && (size_t)A.I * bits / 8 % 16 == 0 && (size_t)A.I * bits % 8 == 0 &&
            ((uintptr_t)A.W & 15) == 0 && ((uintptr_t)A.x & 15) == 0 && A.ldx % 4 == 0 && A.I >= 32;
 }
+// Short rows on many blocks stay with k_lanes16 (nb of its blocks): a block of k_lanes_w fills
+// its pipeline and stages a whole x chunk for a few steps.  The line by k_lanes16 / k_lanes_w,
+// bf16, us a launch: 1024 outputs, 128 tokens (512 blocks) I = 64 8.6 / 9.3, 160 12.2 / 10.8;
+// 4096 outputs, 64 tokens (1024) I = 64 9.8 / 13.9, 256 19.1 / 17.4; 12288 outputs, 128 tokens
+// (6144) I = 64 31 / 59, 320 69 / 85, 384 89 / 87.  On fewer blocks k_lanes16 is behind at any
+// length (64 outputs, 64 tokens, I = 64: 9.0 / 4.8).
+static bool lanes_short(const LanesArgs &A, int64_t nb) {
+    return nb >= 512 && A.I <= (nb / 6 < 224 + nb / 40 ? nb / 6 : 224 + nb / 40);
+}
 
 template <int WK, int DP>
 static void launch_lanes(hipStream_t st, const LanesArgs &A) {
+    const int ts16 = A.S >= 16 ? 16 : A.S >= 8 ? 8 : A.S >= 4 ? 4 : 1;
     if constexpr (WK != WK_I4G) {
-        if (lanes_w_ok(A, WElem<WK>::bits)) {
+        if (lanes_w_ok(A, WElem<WK>::bits) && !lanes_short(A, (int64_t)((A.O + 15) / 16) * ((A.S + ts16 - 1) / ts16))) {
             // tokens per pass: the most (each weight turned once for all of them) that still give
             // 512 blocks, two waves per SIMD -- one alone issues at half rate (bf16 4096 x 4096 at 8
             // tokens, whole call: 66 us with 256 blocks, 58 with 512, 57 with 1024; 24 tokens at
@@ -419,11 +429,10 @@ static void launch_lanes(hipStream_t st, const LanesArgs &A) {
             return;
         }
     }
-    const int ts = A.S >= 16 ? 16 : A.S >= 8 ? 8 : A.S >= 4 ? 4 : 1;
     const dim3 block(256);
-    if (ts == 16) SW_LAUNCH((k_lanes16<WK, DP, 16>), dim3((A.O + 15) / 16, (A.S + 15) / 16), block, 0, st, A);
-    else if (ts == 8) SW_LAUNCH((k_lanes16<WK, DP, 8>), dim3((A.O + 15) / 16, (A.S + 7) / 8), block, 0, st, A);
-    else if (ts == 4) SW_LAUNCH((k_lanes16<WK, DP, 4>), dim3((A.O + 15) / 16, (A.S + 3) / 4), block, 0, st, A);
+    if (ts16 == 16) SW_LAUNCH((k_lanes16<WK, DP, 16>), dim3((A.O + 15) / 16, (A.S + 15) / 16), block, 0, st, A);
+    else if (ts16 == 8) SW_LAUNCH((k_lanes16<WK, DP, 8>), dim3((A.O + 15) / 16, (A.S + 7) / 8), block, 0, st, A);
+    else if (ts16 == 4) SW_LAUNCH((k_lanes16<WK, DP, 4>), dim3((A.O + 15) / 16, (A.S + 3) / 4), block, 0, st, A);
     else SW_LAUNCH((k_lanes16<WK, DP, 1>), dim3((A.O + 15) / 16, A.S), block, 0, st, A);
 }
 

@@ -2,9 +2,10 @@
 16-byte pieces are streamed by waves, everything else takes the general tiles.  Inputs around
 a step (128, 256 or 512 columns by the weight type), an x chunk (512 columns) and the scalar
 tail, outputs around a wave's 4 rows and a block's 16; a weight address off by one element
-takes the general kernel.  With few outputs the streamed kernel runs a token at a time,
-whatever the batch; test_widths has enough of them for its passes of 1, 2, 4 and 8.  All bit
-for bit the oracle's, whose matmuls are pinned to the compiled reference."""
+takes the general kernel, and so do short rows of many outputs.  With few outputs the streamed
+kernel runs a token at a time, whatever the batch; test_widths has enough of them for its
+passes of 1, 2, 4 and 8.  All bit for bit the oracle's, whose matmuls are pinned to the
+compiled reference."""
 import numpy as np
 import pytest
 
@@ -89,18 +90,38 @@ def _width(O, S):
     return ts
 
 
+def _short(O, S, I):
+    """rows too short, for that many blocks, to be streamed"""
+    ts = 16 if S >= 16 else 8 if S >= 8 else 4 if S >= 4 else 1
+    nb = -(-O // 16) * -(-S // ts)
+    return nb >= 512 and I <= min(nb // 6, 224 + nb // 40)
+
+
 WIDE_O = 8195                                         # 513 blocks a pass: every width is reached
 WIDE_S = [1, 2, 3, 4, 7, 8, 9, 17]                    # full passes, and passes with tokens past the batch
 
 
-@pytest.mark.parametrize("kind,I", [("bf16", 32), ("bf16", 160), ("bf16", 536), ("bf16", 1056),
-                                    ("bf16_rx", 32), ("bf16_rx", 160), ("bf16_rx", 544), ("bf16_rx", 1056),
-                                    ("q8", 32), ("q8", 272), ("q8", 528), ("q8", 1040),
-                                    ("q4", 32), ("q4", 160), ("q4", 544), ("q4", 1056)])
+@pytest.mark.parametrize("kind,I", [("bf16", 288), ("bf16", 536), ("bf16", 1056),
+                                    ("bf16_rx", 288), ("bf16_rx", 544), ("bf16_rx", 1056),
+                                    ("q8", 272), ("q8", 528), ("q8", 1040),
+                                    ("q4", 288), ("q4", 544), ("q4", 1056)])
 def test_widths(be, orc, kind, I):
     """each width of the streamed kernel on full and partial steps and chunks"""
+    assert [_width(WIDE_O, S) for S in WIDE_S] == [1, 2, 4, 4, 4, 8, 8, 8]
+    assert not any(_short(WIDE_O, S, I) for S in WIDE_S)
+    _against_oracle(be, orc, kind, I)
+
+
+@pytest.mark.parametrize("kind,I", [("bf16", 32), ("bf16", 160), ("bf16_rx", 32), ("bf16_rx", 160),
+                                    ("q8", 32), ("q8", 160), ("q4", 32), ("q4", 160)])
+def test_short_rows(be, orc, kind, I):
+    """rows of whole pieces on both sides of the line to the general kernel"""
+    assert {_short(WIDE_O, S, I) for S in WIDE_S} == ({True} if I == 32 else {True, False})
+    _against_oracle(be, orc, kind, I)
+
+
+def _against_oracle(be, orc, kind, I):
     O = WIDE_O
-    assert [_width(O, S) for S in WIDE_S] == [1, 2, 4, 4, 4, 8, 8, 8]
     rng = np.random.default_rng(I * 149 + len(kind))
     sc = rng.uniform(1e-3, 2e-3, O).astype(np.float32)
     if kind == "q8":
@@ -123,8 +144,8 @@ def test_widths(be, orc, kind, I):
 
 @pytest.mark.parametrize("S", [8 * 65535, 8 * 65535 + 1])
 def test_most_tokens(be, orc, S):
-    """the last row count whose passes of 8 fit a grid's second dimension (65535), and one
-    more, which the general kernel's passes of 16 take"""
+    """the last row count whose passes of 8 tokens would fit a grid's second dimension (65535),
+    and one more (such short rows take the general kernel's passes of 16 either way)"""
     I = 32
     rng = np.random.default_rng(S)
     q = rng.integers(-127, 128, (1, I)).astype(np.int8)
