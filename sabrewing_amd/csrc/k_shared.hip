@@ -350,11 +350,16 @@ int sw_launch_sh_glu(hipStream_t st, const uint16_t *Wg, const uint16_t *Wu, con
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// The down on its own: the split-K blocks while the batch is one tile of k_sh_down_mf's
-// (C2 at 40 / 64 / 96 / 125 tokens: 16 / 21 / 29 / 37 us split, 24 / 24 / 23 / 24 in tiles)
+// The down on its own: the split-K blocks while the batch is one tile of k_sh_down_mf's, and
+// up to 128 tokens while they run in one round on the CUs, or in two where K is long (a tile's
+// time is its serial loop over K; D / 16 x S / 32 split blocks against D / 128 x 2 tiles).  us
+// split / tiles, 128 tokens: D = 1024 (256 blocks) Is = 512 8.2 / 11.6, 2048 14 / 32; D = 2048
+// (512) Is = 512 15 / 11.5, 1024 15 / 18, 2048 27 / 32; D = 4096 (1024) Is = 1024 30 / 18.6
 int sw_launch_sh_down(hipStream_t st, const uint16_t *Wd, const uint16_t *hp, int S, int Is, int D, float *out) {
     if (S <= 0 || D % 128 || Is % (SHB_NG * SH_RG) || !sh_shape_ok(Is)) return -1;
-    if (S <= SHB_TOK) return launch_sk<0>(st, Wd, nullptr, hp, S, Is, D, out);
+    const int64_t blocks = (int64_t)sh_sk_rows(0, D) * sh_sk_cols(S, sh_sk_nc(0, S));
+    if (S <= SHB_TOK || (S <= SH_SK_MAX_S && blocks <= (Is >= 1024 ? 512 : 256)))
+        return launch_sk<0>(st, Wd, nullptr, hp, S, Is, D, out);
     const dim3 grid((unsigned)(D / 128 * ((S + SHB_TOK - 1) / SHB_TOK)));
     SW_LAUNCH(k_sh_down_mf, grid, dim3(256), 0, st, Wd, hp, S, Is, D, out);
     return hipGetLastError() == hipSuccess ? 0 : -1;

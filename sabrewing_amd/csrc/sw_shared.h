@@ -256,8 +256,8 @@ struct ShSkArgs {
 };
 #define SH_SK_NT 512
 // batches up to this many tokens take these blocks inside other launches; on its own the
-// gate_up splits K up to here too (these blocks or k_sh_glu_skr's), the down up to 64 tokens
-// (sw_launch_sh_glu, sw_launch_sh_down)
+// gate_up splits K up to here too (these blocks or k_sh_glu_skr's), the down where its grid is
+// small (sw_launch_sh_glu, sw_launch_sh_down)
 #define SH_SK_MAX_S 128
 // column tiles of 16 tokens per block: gate_up 1 up to 32 tokens (the grid then fills
 // the chip), else 2; the down's segments are short: always 2

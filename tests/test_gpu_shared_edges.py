@@ -12,8 +12,9 @@ from sabrewing_amd.backend import DeviceLayer, desc_of
 pytestmark = pytest.mark.gpu
 MFMA = 2          # the experts on the MFMA: the shared expert runs in launches of its own
 
-# (D, Is): segments of 1 group; 4 segments of 3 groups; 4 segments of 9 in the down
-SHAPES = [(256, 1024), (384, 1024), (256, 1152)]
+# (D, Is): segments of 1 group; 4 segments of 3 groups; 4 segments of 9 in the down; a down of
+# 65 to 128 tokens in tiles, and one whose K split runs in two rounds on the CUs
+SHAPES = [(256, 1024), (384, 1024), (256, 1152), (1536, 512), (1536, 1024)]
 
 
 @pytest.mark.parametrize("D,Is", SHAPES)
