@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
+#include <math.h>
 
 typedef _Float16 sw_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 sw_half2 __attribute__((ext_vector_type(2)));
@@ -177,22 +178,49 @@ __host__ __device__ inline int sw_npass_max(int T, int E, int tt) { return (T + 
 // at 4.4 725 / 694, at 5 778 / 704, at 7 1,049 / 745; C1 at 4 108 / 103, at 6 139 / 106;
 // D = 2048, I = 512, E = 256 at 4 211 / 196; C5 at 4 909 / 901, at 4.75 1,030 / 926.
 __host__ __device__ inline bool sw_mf_wins(int64_t T, int64_t G) { return 4 * T >= 19 * G; }
-// tokens per tile of the MFMA launches: 16 (four waves per SIMD) up to 9 rows a group, 32 up
-// to 22, else 64 (each weight expanded once for four columns of tokens).  Per layer step with
-// 16 / 32 / 64: C2 at 5 rows a group 704 / 722 / 804 us, at 9 829 / 822 / 936, at 10 848 / 821
-// / 951, at 20 1,248 / 1,119 / 1,110, at 27 1,440 / 1,242 / 1,211, at 40 1,889 / 1,722 / 1,460;
-// C1 at 20 181 / 145 / 152, at 25 212 / 201 / 167; C5 at 22 1,667 / 1,439 / 1,433.
-// Few blocks: a launch has tiles x I / 128 (gate_up) or D / 256 (down) blocks, and a
-// block alone on its CU takes 46 us with one column (gate_up, K = 4096), 66 with two, 85 with
-// three, 121 with four; so while a tile half as wide still gives every block a CU of its own,
-// it is taken: below 112 blocks of 256 CUs, not 128, for the groups that end in a partial tile.
-// gate_up + down with 16 / 32 / 64: D = 4096, I = 1024, a group of 64 rows 62 / 88 / 159 us, 4
-// of 64 78 / 92 / 164, 4 of 128 136 / 117 / 170; D = 5120, I = 1536, 4 of 64 86 / 106 / 165.
+// tokens per tile of the MFMA launches, from T packed rows in G groups.  Where the launches
+// fill the chip many times over: 16 (four waves per SIMD) up to 9 rows a group, 32 up to 22, else
+// 64 (each weight expanded once for four columns of tokens).  Per layer step with 16 / 32 / 64:
+// C2 at 5 rows a group 704 / 722 / 804 us, at 9 829 / 822 / 936, at 10 848 / 821 / 951, at 20
+// 1,248 / 1,119 / 1,110, at 27 1,440 / 1,242 / 1,211, at 40 1,889 / 1,722 / 1,460; C1 at 20 181 /
+// 145 / 152, at 25 212 / 201 / 167; C5 at 22 1,667 / 1,439 / 1,433.
+// Few or short blocks: narrower where that should save 5 % by the rounds of blocks on the 256
+// CUs times a block's time, which is 2, 2.5 or 3 us to fill and drain plus, per 4096 inputs and
+// by its columns, 46 / 50, 66 / 62, 68, 90, 125 us (blocks alone on their CUs).  gate_up + down
+// with 16 / 32 / 64: D = 4096, I = 1024, a group of 64 rows 62 / 88 / 159 us, 4 of 64 78 / 92 /
+// 164, 4 of 128 136 / 117 / 170; D = 5120, I = 1536, 4 of 64 86 / 106 / 165; layer steps: D =
+// 2048, I = 256, 56 groups of 27 78 / 86 / 98, D = 896, I = 512, 40 of 82 103 / 102 / 137.  Over
+// 469 measured shapes the choice is 2.3 % behind the best of the three on average, at most 36 %
+// (the tiles of an average group are estimated), against 33 % on average by the rows alone.
+// the tiles of at most tt tokens of a group of n on average, its size spread as a Poisson's
+inline double sw_mf_parts(double n, int tt) {
+    const double s = sqrt(2 * n);
+    int64_t k = n > 4 * s ? (int64_t)((n - 4 * s) / tt) : 0;
+    double e = 1.0 + (double)k;
+    for (k++; (double)k * tt < n + 4 * s; k++) e += 0.5 * erfc(((double)k * tt + 0.5 - n) / s);
+    return e;
+}
 inline int sw_mf_cols(int64_t T, int64_t G, int D, int I) {
-    int tt = T <= 9 * G ? 16 : T <= 22 * G ? 32 : SW_MF_TT;
-    const int64_t nb = I / 128 < (D + 255) / 256 ? I / 128 : (D + 255) / 256;
-    while (tt > 16 && (T > G * tt ? (T + tt - 1) / tt : G) * nb < 112) tt >>= 1;
-    return tt;
+    const int top = T <= 9 * G ? 16 : T <= 22 * G ? 32 : SW_MF_TT;
+    if (top == 16) return top;
+    const double n = (double)T / G, cols = G * sw_mf_parts(n, 16);
+    int best = top;
+    double limit = 0;
+    for (int tt = top; tt >= 16; tt >>= 1) {
+        static const double fill[3] = {2, 2.5, 3}, col[3][4] = {{46}, {50, 66}, {62, 68, 90, 125}};
+        const int w = tt == 16 ? 0 : tt == 32 ? 1 : 2, nc = tt / 16;
+        const double tiles = G * sw_mf_parts(n, tt), x = cols / tiles < nc ? cols / tiles : nc;
+        const int lo = x < nc ? (int)x : nc > 1 ? nc - 1 : 1;           // columns a tile, between lo and lo + 1
+        const double c = nc == 1 ? col[w][0] : col[w][lo - 1] + (x - lo) * (col[w][lo] - col[w][lo - 1]);
+        double t = 0;
+        for (int l = 0; l < 2; l++) {
+            const double rounds = ceil(tiles * (l ? (D + 255) / 256 : I / 128) / 256 - 0.02);
+            t += (rounds < 1 ? 1 : rounds) * (fill[w] + (l ? I : D) / 4096.0 * c);
+        }
+        if (tt == top) limit = 0.95 * t;
+        else if (t < limit) { limit = t; best = tt; }
+    }
+    return best;
 }
 // the MFMA tiles of a group of n tokens, at most tt each: ceil(n / tt) of them, each of the
 // same whole number of 16-token columns (80 tokens in 64s: 48 + 32, not 64 + 16 -- a tail

@@ -138,13 +138,13 @@ def test_expert_group_one_row_each(coli, be, orc, gs):
 
 @pytest.mark.parametrize("gs", [0, 32])
 @pytest.mark.parametrize("ids,rows,tt", [([3, 1, 4, 0], [40, 70, 9, 130], 16),
-                                         ([3, 1, 4, 0, 5, 2] * 5, [12, 9, 32, 15, 17, 10] * 5, 32),
-                                         ([3, 1, 4, 0, 5, 2] * 5, [40, 70, 9, 130, 1, 64] * 5, 64)],
+                                         ([3, 1, 4, 0, 5, 2] * 10, [12, 9, 32, 15, 17, 10] * 10, 32),
+                                         ([3, 1, 4, 0, 5, 2] * 6, [40, 70, 9, 130, 1, 64] * 6, 64)],
                          ids=["tiles16", "tiles32", "tiles64"])
 def test_prefill_group_on_the_mfma(coli, be, orc, gs, ids, rows, tt):
     """groups averaging >= 8 rows take the f16 MFMA GEMMs (partial tiles, groups over several
     tiles; 16-token tiles for four groups, which are few blocks, 32- and 64-token tiles for
-    30): still each row's lag expert output bit for bit"""
+    60 and 36): still each row's lag expert output bit for bit"""
     assert tile_width(rows, D, I) == tt
     L = layer(orc, gs, seed=21)
     ex = Experts(coli, L, gs)
