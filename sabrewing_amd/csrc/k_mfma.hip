@@ -37,21 +37,22 @@
 //
 // What bounds it: no one unit.  A step is 2 MFMAs, 4 conversions (one fma each), 4 products of
 // scale and factor, 4 terms, 4 sums on average, and its share of the expansion (9 operations
-// per 8 weights): a quad of 4, 3, 2 or 1 columns has 603, 483, 363 or 247 VALU instructions
+// per 8 weights): a quad of 4, 3, 2 or 1 columns has 599, 479, 359 or 243 VALU instructions
 // beside 64, 48, 32 or 16 MFMAs.  VALU issue is the largest part, but 12 % more instructions
 // in the loop took 3 % longer at 64 tokens and 7 % more 0.6-1.5 % at 16; at 64 tokens the
-// waves, two per SIMD, spend 25-30 % of their time waiting (LDS reads, 1 KB per step for two
-// row tiles, and a barrier per chunk).  (Those instructions round every term before it is added.  Acc
-// times s, with the power of two applied by the fma of the add, had 8 fewer per quad, row tile
-// and column: C2 S = 2048 gate_up 1,456 against 1,505 us, S = 181 412 against 414.  It left
-// dot8's bits where s * xf is no normal number, acc * s overflows or a term does.)
-// 16 tokens (NT = 1) fit 128 registers, four waves per SIMD; 64 take 256, two, and spill:
-// gate_up 22, down 56 registers (group scales of 32), paid per run and row block but for one
-// reload a quad.
+// waves, two per SIMD, spend 26 % of their time waiting (LDS reads, 1 KB per step for two
+// row tiles, and a barrier per chunk).  (Those instructions round every term before it is
+// added.  Acc times s, with the power of two applied by the fma of the add, had 8 fewer per
+// quad, row tile and column, but left dot8's bits where s * xf is no normal number, acc * s
+// overflows or a term does.)  A run's four quads stand in a line: as two loops of two, every
+// pair began with an add to -0, and at 64 tokens a register reloaded in each quad made its
+// wait drain the loads in flight (a step of C2, S = 2048, 4.5 % longer, S = 181 2.4 %, of C1, S
+// = 333, 5.5 %).  16 tokens (NT = 1) fit 128 registers, four waves per SIMD; 64 take 256, two,
+// and spill 13 (gate_up) and 47 (down, group scales of 32), reloaded once or a few times a run.
 // Expanding in every wave from registers replaced weights expanded once per block into LDS,
 // whose reads (1 KB per row tile and group) and barriers (one per chunk over 16 waves) bounded
-// the loop: C2 S = 2048 gate_up 1,783 -> 1,505 us, down 990 -> 862; S = 181 571 -> 414 and
-// 314 -> 235; C1 S = 333 gate_up 148 -> 140, down 78 -> 82.
+// the loop: C2 S = 2048 gate_up 1,754 -> 1,425 us, down 963 -> 786; S = 181 568 -> 400 and 313
+// -> 224; C1 S = 333 147 -> 131 and 78 -> 76.
 #include "sw_hip.h"
 #include "sw_gate.h"
 
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
         // chunk's digits -- are issued at its top and waited for at the next one's or at the
         // chunk's end, a whole quad's work later: issued at its end, the next top's wait for
         // the (older) weights would drain them too
-        auto quad = [&](int rb, int qc, sw_f32x4 (&acc)[2][NA]) {
+        auto quad = [&](auto FIRST, int rb, int qc, sw_f32x4 (&acc)[2][NA]) {   // FIRST: acc starts here
             // the quad's operands: 4 groups of both row tiles, then the next quad's loads
             // (expanded once for several columns; for a single one group by group, in registers)
             sw_half8 a[2][NA > 1 ? 4 : 1];
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
                 if (g == 0 || g == 2) asm volatile("" : "+v"(h[t]));
                 else asm volatile("" : "+v"(q[t]));
                 if (t == 1 && (i >> 1) + 2 < NS / 2) fetch((i >> 1) + 2, op[(i >> 1) & 1]);
-                if (g == 3) acc[t][c] = acc[t][c] + q[t];
+                if (g == 3) acc[t][c] = decltype(FIRST)::v ? q[t] : acc[t][c] + q[t];
                 __builtin_amdgcn_sched_barrier(0);
             }
             // the chunk's last quad: the next chunk into the other buffer (read by no wave since
@@ -431,7 +432,7 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
 #pragma unroll
                 for (int c = 0; c < NA; c++) v[t][c] = sw_f32x4{x, x, x, x};
         };
-        // (sums start from -0, the identity of f32 addition: the first term's bits as they are)
+        // (y starts from -0, the identity of f32 addition: the first run's bits as they are)
         for (int rbi = 0; rbi < rbper; rbi++) {
             const int rb = rbf + rbi;
             sw_f32x4 y[2][NA];
@@ -440,13 +441,13 @@ __global__ __launch_bounds__(MF_NTH, NT == 1 ? 4 : 2) void k_mf(MfArgs A) {
             for (int r0 = 0; r0 < NC; r0 += 4) {
                 // a run: (q0 + q1) + (q2 + q3), a short last run padded with +0 terms
                 sw_f32x4 ra[2][NA], rv[2][NA];
-                fill(ra, -0.f);
-#pragma unroll 1
-                for (int qc = r0; qc < min(r0 + 2, NC); qc++) quad(rb, qc, ra);
+                quad(MfIc<1>{}, rb, r0, ra);
+                if (r0 + 1 < NC) quad(MfIc<0>{}, rb, r0 + 1, ra);
                 if (NQ == 4) {
-                    fill(rv, r0 + 2 < NC ? -0.f : 0.f);
-#pragma unroll 1
-                    for (int qc = r0 + 2; qc < min(r0 + 4, NC); qc++) quad(rb, qc, rv);
+                    if (r0 + 2 < NC) {
+                        quad(MfIc<1>{}, rb, r0 + 2, rv);
+                        if (r0 + 3 < NC) quad(MfIc<0>{}, rb, r0 + 3, rv);
+                    } else fill(rv, 0.f);
                     if (r0 + 4 > NC) {
 #pragma unroll
                         for (int t = 0; t < 2; t++)

@@ -174,24 +174,24 @@ __host__ __device__ inline int sw_npass_max(int T, int E, int tt) { return (T + 
 // The MFMA against dot8 for T packed rows in G groups: from 4.75 rows a group.  dot8's time
 // grows with the rows (24 dots per weight group and row), the MFMA's hardly does up to 16.
 // The two cross between 3.5 and 4.5 rows, by half a row differently from run to run; the line
-// lies above that.  Per layer step, dot8 against the MFMA: C2 at 3.5 rows a group 617 / 678 us,
-// at 4.4 725 / 694, at 5 778 / 704, at 7 1,049 / 745; C1 at 4 108 / 103, at 6 139 / 106;
-// D = 2048, I = 512, E = 256 at 4 211 / 196; C5 at 4 909 / 901, at 4.75 1,030 / 926.
+// lies above that.  Per layer step, dot8 against the MFMA: C2 at 3.5 rows a group 605 / 660 us,
+// at 4.4 704 / 677, at 5 766 / 681, at 7 1,041 / 730; C1 at 4 107 / 97, at 6 137 / 102; D = 2048,
+// I = 512, E = 256 at 4 211 / 191; C5 at 4 901 / 878, at 4.75 1,013 / 900.
 __host__ __device__ inline bool sw_mf_wins(int64_t T, int64_t G) { return 4 * T >= 19 * G; }
 // tokens per tile of the MFMA launches, from T packed rows in G groups.  Where the launches
 // fill the chip many times over: 16 (four waves per SIMD) up to 9 rows a group, 32 up to 22, else
 // 64 (each weight expanded once for four columns of tokens).  Per layer step with 16 / 32 / 64:
-// C2 at 5 rows a group 704 / 722 / 804 us, at 9 829 / 822 / 936, at 10 848 / 821 / 951, at 20
-// 1,248 / 1,119 / 1,110, at 27 1,440 / 1,242 / 1,211, at 40 1,889 / 1,722 / 1,460; C1 at 20 181 /
-// 145 / 152, at 25 212 / 201 / 167; C5 at 22 1,667 / 1,439 / 1,433.
+// C2 at 5 rows a group 681 / 714 / 795 us, at 9 809 / 813 / 923, at 10 826 / 818 / 948, at 20
+// 1,223 / 1,075 / 1,094, at 27 1,414 / 1,183 / 1,178, at 40 1,851 / 1,646 / 1,399; C1 at 20 176 /
+// 140 / 149, at 25 204 / 193 / 164; C5 at 22 1,636 / 1,373 / 1,409.
 // Few or short blocks: narrower where that should save 5 % by the rounds of blocks on the 256
 // CUs times a block's time, which is 2, 2.5 or 3 us to fill and drain plus, per 4096 inputs and
-// by its columns, 46 / 50, 66 / 62, 68, 90, 125 us (blocks alone on their CUs).  gate_up + down
-// with 16 / 32 / 64: D = 4096, I = 1024, a group of 64 rows 62 / 88 / 159 us, 4 of 64 78 / 92 /
-// 164, 4 of 128 136 / 117 / 170; D = 5120, I = 1536, 4 of 64 86 / 106 / 165; layer steps: D =
-// 2048, I = 256, 56 groups of 27 78 / 86 / 98, D = 896, I = 512, 40 of 82 103 / 102 / 137.  Over
-// 469 measured shapes the choice is 2.3 % behind the best of the three on average, at most 36 %
-// (the tiles of an average group are estimated), against 33 % on average by the rows alone.
+// by its columns, 45 / 50, 64 / 62, 68, 85, 115 us (blocks alone on their CUs).  gate_up + down
+// with 16 / 32 / 64: D = 4096, I = 1024, a group of 64 rows 60 / 84 / 140 us, 4 of 64 77 / 88 /
+// 146, 4 of 128 135 / 112 / 152; D = 5120, I = 1536, 4 of 64 85 / 104 / 159; layer steps: D =
+// 2048, I = 256, 56 groups of 27 76 / 83 / 93, D = 896, I = 512, 40 of 82 102 / 98 / 128.  Over
+// 469 measured shapes the choice is 1.8 % behind the best of the three on average, at most 33 %
+// (the tiles of an average group are estimated), against 31 % on average by the rows alone.
 // the tiles of at most tt tokens of a group of n on average, its size spread as a Poisson's
 inline double sw_mf_parts(double n, int tt) {
     const double s = sqrt(2 * n);
@@ -207,7 +207,7 @@ inline int sw_mf_cols(int64_t T, int64_t G, int D, int I) {
     int best = top;
     double limit = 0;
     for (int tt = top; tt >= 16; tt >>= 1) {
-        static const double fill[3] = {2, 2.5, 3}, col[3][4] = {{46}, {50, 66}, {62, 68, 90, 125}};
+        static const double fill[3] = {2, 2.5, 3}, col[3][4] = {{45}, {50, 64}, {62, 68, 85, 115}};
         const int w = tt == 16 ? 0 : tt == 32 ? 1 : 2, nc = tt / 16;
         const double tiles = G * sw_mf_parts(n, tt), x = cols / tiles < nc ? cols / tiles : nc;
         const int lo = x < nc ? (int)x : nc > 1 ? nc - 1 : 1;           // columns a tile, between lo and lo + 1

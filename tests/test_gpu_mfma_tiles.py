@@ -49,7 +49,7 @@ def tile_width(sizes, D, I):
         return top
     n = T / G
     cols, best, limit = G * _parts(n, 16), top, 0.0
-    for tt, fill, col in ((64, 3, (62, 68, 90, 125)), (32, 2.5, (50, 66)), (16, 2, (46,))):
+    for tt, fill, col in ((64, 3, (62, 68, 85, 115)), (32, 2.5, (50, 64)), (16, 2, (45,))):
         if tt > top:
             continue
         tiles = G * _parts(n, tt)
@@ -110,7 +110,7 @@ def _row_blocks(D, I, sizes):
 
 # (D, groups, rows per group, tile width, row blocks per block): D of 3.5 and 7.5 row blocks
 MANY = [(1920, 540, (1, 9), 16, 4), (1920, 280, (1, 9), 16, 2), (1920, 560, (8, 23), 32, 4), (1920, 260, (8, 23), 32, 2),
-        (1920, 560, (20, 40), 64, 4), (1920, 280, (17, 33), 64, 2), (896, 640, (8, 23), 32, 2), (896, 540, (1, 9), 16, 2)]
+        (1920, 560, (20, 40), 64, 4), (1920, 256, (24, 48), 64, 2), (896, 640, (8, 23), 32, 2), (896, 540, (1, 9), 16, 2)]
 
 
 @pytest.mark.parametrize("gs", [0, 32])
