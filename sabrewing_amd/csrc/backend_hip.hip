@@ -260,7 +260,7 @@ static int grouped_host(float *outh, const float *x, int S, const void *gu_q, co
     if (D <= 0 || I <= 0 || G <= 0 || S <= 0) return -1;
     const int T = S * K;
     // the MFMA kernels for prefill-sized groups: tiles of up to tt tokens, listed here
-    const int tt = sw_mf_cols(T, G, D, I);
+    const int tt = sw_mf_cols(T, G, D, I, gcnt);
     int ntile = 0;
     for (int i = 0; i < G; i++) ntile += (gcnt[i] + tt - 1) / tt;
     const bool mf = G < 1024 && T < (1 << 21) && use_mfma(T, G, D, I);

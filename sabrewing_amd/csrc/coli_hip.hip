@@ -235,7 +235,7 @@ int group_sync(const Groups &G, float *y, const float *x) {
     if (!select_ctx(c)) return 0;
     const int T = G.total;
     const bool mf = use_mf(G);
-    const int tt = sw_mf_cols(T, G.count, G.D, G.I);       // tokens per MFMA tile
+    const int tt = sw_mf_cols(T, G.count, G.D, G.I, G.cnt.data());   // tokens per MFMA tile
     std::vector<int> items;
     if (mf) {
         for (int g = 0; g < G.count; g++)

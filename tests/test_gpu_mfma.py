@@ -79,7 +79,7 @@ def test_mfma_multi_tile_groups(be, orc, E, K, S_):
     # per-token (decode path) for a few streams
     single = np.stack([block(be, cfg, dl, x[s:s + 1], base[s:s + 1], AUTO)[0] for s in (0, 199, 399)])
     dl.free()
-    assert max(gcnt[:G]) > 64 and tile_width([int(n) for n in gcnt[:G]], cfg.D, cfg.I) == (16 if E == 8 else 64)
+    assert max(gcnt[:G]) > 64 and tile_width([int(n) for n in gcnt[:G]], cfg.D, cfg.I, known=False) == (16 if E == 8 else 64)
     assert np.array_equal(bits(got_m), bits(got_d))
     assert np.array_equal(bits(got_m[[0, 199, 399]]), bits(single))
     assert errs(got_m, orc.moe_block_rows(synth.desc_of(cfg), L, x, base), base) <= TOL

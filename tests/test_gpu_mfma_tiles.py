@@ -40,21 +40,21 @@ def _parts(n, tt):
     return e
 
 
-def tile_width(sizes, D, I):
+def tile_width(sizes, D, I, known=True):
     """the launch rule (sw_mf_cols): by the average group, narrower where the rounds of blocks
-    on the CUs times a block's time say so"""
+    on the CUs times a block's time say so; known: the host knows the groups' sizes"""
     T, G = sum(sizes), len(sizes)
     top = 16 if T <= 9 * G else 32 if T <= 22 * G else 64
     if top == 16:
         return top
-    n = T / G
-    cols, best, limit = G * _parts(n, 16), top, 0.0
+    parts = lambda tt: sum(-(-n // tt) for n in sizes) if known else G * _parts(T / G, tt)
+    cols, best, limit = parts(16), top, 0.0
     for tt, fill, col in ((64, 3, (62, 68, 85, 115)), (32, 2.5, (50, 64)), (16, 2, (45,))):
         if tt > top:
             continue
-        tiles = G * _parts(n, tt)
+        tiles = parts(tt)
         c = float(np.interp(cols / tiles, range(1, tt // 16 + 1), col))
-        t = sum(max(1, math.ceil(tiles * nb / 256 - 0.02)) * (fill + K / 4096 * c) for K, nb in ((D, I // 128), (I, -(-D // 256))))
+        t = sum(max(1, math.ceil(tiles * nb / 256 - (0 if known else 0.01))) * (fill + K / 4096 * c) for K, nb in ((D, I // 128), (I, -(-D // 256))))
         if tt == top:
             limit = 0.95 * t
         elif t < limit:
@@ -109,7 +109,7 @@ def _row_blocks(D, I, sizes):
 
 
 # (D, groups, rows per group, tile width, row blocks per block): D of 3.5 and 7.5 row blocks
-MANY = [(1920, 540, (1, 9), 16, 4), (1920, 280, (1, 9), 16, 2), (1920, 560, (8, 23), 32, 4), (1920, 260, (8, 23), 32, 2),
+MANY = [(1920, 540, (1, 9), 16, 4), (1920, 280, (1, 9), 16, 2), (1920, 560, (8, 23), 32, 4), (1920, 360, (8, 23), 32, 2),
         (1920, 560, (20, 40), 64, 4), (1920, 256, (24, 48), 64, 2), (896, 640, (8, 23), 32, 2), (896, 540, (1, 9), 16, 2)]
 
 
